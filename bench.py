@@ -157,8 +157,7 @@ def time_to_target(n_sessions, batch_sessions, lr, max_epochs, seed=5):
     curve = []
     reached = None
     # Minibatch steps have fewer sessions to spread over the chip than a full
-    # EM pass: 4096-session work items were the fastest of 1024-8192 for them
-    # (8192, the default, for EM).
+    # EM pass: 4096-session work items were the fastest of 1024-8192 for them.
     with ClickModel(DBN, batches=batches, item_sessions=ADAM_ITEM_SESSIONS) as cm:
         cm.init_from_dataset(ds)
         cm.set_test_set(test)
@@ -183,7 +182,7 @@ def time_to_target(n_sessions, batch_sessions, lr, max_epochs, seed=5):
     return {
         "workload": f"DBN, {n_sessions} synthetic sessions ({ds.n_train} train), 1M Zipf(1.1) queries; Adam lr {lr}, "
                     f"{batches} minibatches of whole query groups (~{batch_sessions} sessions), log-prior on, "
-                    f"{ADAM_ITEM_SESSIONS}-session work items (EM: 8192)",
+                    f"{ADAM_ITEM_SESSIONS}-session work items",
         "target_heldout_ll": target,
         "threshold": "held-out LL at least EM's 50-iteration LL minus 1e-4 relative",
         "em_ms": em_ms,
@@ -443,8 +442,7 @@ def main():
                    "work_items": lay["n_items"], "autotune": tune},
         "roofline": {"bound": "hbm", "achieved": achieved / 1e9, "peak": HBM_PEAK / 1e9, "unit": "GB/s",
                      "frac": achieved / HBM_PEAK, "traffic": traffic, "traffic_source": traffic_src,
-                     "kernel": ("em_window_persistent_kernel" if segmented and opts.get("persistent", True)
-                                and opts.get("block", 256) == 256 else "em_item_kernel"),
+                     "kernel": "em_item_kernel",
                      "bytes_per_launch": item_bytes,
                      "layout_bytes_per_launch": layout_bytes,
                      "layout_frac": layout_bytes / (kt["ms_estep"] * 1e-3) / HBM_PEAK,

@@ -42,23 +42,23 @@ typedef enum {
 enum {
     /* 0 = deterministic segmented reduction (default), 1 = float atomics. */
     MC_OPT_REDUCE_MODE = 0,
-    /* Target sessions per workgroup work item (default 8192). */
+    /* Target sessions per workgroup work item (default: chosen for the
+     * training set, 256 to 16384; 8192 in the float-atomic mode). */
     MC_OPT_ITEM_SESSIONS = 1,
     /* Per-qd accumulator window per work item, in entries (default 1280). */
     MC_OPT_ITEM_WINDOW = 2,
     /* 1 = reorder sessions inside each work item by length, then last-click
      * rank, so that wavefronts run uniform chains (default 1). */
     MC_OPT_SORT_BY_LCR = 3,
-    /* Workgroup size of the E/M kernel: 64, 128, 256 or 512 (default 256). */
+    /* Workgroup size of the E/M kernel: 64, 128, 256 or 512 (default: 256 or
+     * 512, chosen for the model and the training set). */
     MC_OPT_BLOCK = 4,
     /* 1 = sessions that are the only session of their query (and show
      * distinct documents) update their entries directly, without a
      * reduction (default 0). */
     MC_OPT_DIRECT = 5,
-    /* 1 = window items run in one persistent kernel: each resident
-     * workgroup walks a fixed stride of items and prefetches its next item
-     * (default 1; needs MC_OPT_BLOCK 256 and a window of at most 1280
-     * entries). */
+    /* No effect (accepted for callers that set it): every work item runs as
+     * one workgroup. */
     MC_OPT_PERSISTENT = 6,
     /* Minibatches of the gradient path (mc_adam_steps): the query-sorted
      * training set is cut into this many runs of whole query groups of about
@@ -77,12 +77,11 @@ enum {
      * constant bases at init, so visiting them changes no result.  The
      * sessions stay on the device for the gradient path.  0 = visit them. */
     MC_OPT_SKIP_CONSTANT = 9,
-    /* 1 = when the window kernel (persistent or one workgroup per item) is
-     * an iteration's only E-step launch, it also runs the M-step: the
-     * workgroup that adds the last slice of a query group split over several
-     * work items finalises the group's entries, and the last workgroup to
-     * finish the shared tables, so no merge kernel is launched (default 1).
-     * Same results. */
+    /* 1 = when every work item of an iteration is a window item, the window
+     * kernel also runs the M-step: the workgroup that adds the last slice of
+     * a query group split over several work items finalises the group's
+     * entries, and the last workgroup to finish the shared tables, so no
+     * merge kernel is launched (default 1).  Same results. */
     MC_OPT_FUSED_MERGE = 10
 };
 enum { MC_REDUCE_SEGMENTED = 0, MC_REDUCE_ATOMIC = 1 };
@@ -284,9 +283,9 @@ mc_status mc_get_session_formats(const mc_model* m, int64_t* n_packed, int64_t* 
  * candidate itself) and the fastest found on exit.  Each candidate is
  * measured as `iterations` EM iterations replayed from a graph on `device`
  * on this training set (arguments as mc_init_parameters): the reduction mode
- * first, then sessions per work item (2048..16384, i.e. sessions per lane),
- * the LDS window, the launch shape (persistent kernel, or one workgroup
- * of 256 or 512 lanes per item) and the session format (MC_OPT_PACKED).  *best_ms_per_iter and *n_trials report the
+ * first, then sessions per work item (512..16384, i.e. sessions per lane),
+ * the LDS window, the lanes per work item (256 or 512) and the session
+ * format (MC_OPT_PACKED).  *best_ms_per_iter and *n_trials report the
  * winner's time and the number of candidates measured. */
 mc_status mc_autotune(int model_type, int device, int64_t n, const int32_t* query, const int32_t* pidx,
                       const uint8_t* clicks, const uint8_t* len, int64_t n_qd, int iterations, int64_t* options,

@@ -220,12 +220,15 @@ int main(int argc, char** argv) {
                                        tr.clicks.data(), nullptr, ds.n_qd(), 5, opts, &ms, &trials));
             std::cout << "\nAutotune (" << trials << " candidates): reduce-mode " << opts[MC_OPT_REDUCE_MODE]
                       << ", item-sessions " << opts[MC_OPT_ITEM_SESSIONS] << ", window " << opts[MC_OPT_ITEM_WINDOW]
-                      << ", persistent " << opts[MC_OPT_PERSISTENT] << ", block " << opts[MC_OPT_BLOCK] << ": " << ms
+                      << ", block " << opts[MC_OPT_BLOCK] << ": " << ms
                       << " ms/iteration" << std::endl;
         }
         if (config.fit == "adam") opts[MC_OPT_BATCHES] = std::max(1, config.batches);
         mclicks::ClickModel cm(config.model_type, 0);
-        for (int o = 0; o < MC_N_OPTIONS; o++) cm.set_option(o, opts[o]);
+        // Options that nothing has chosen keep the library's defaults, which
+        // it picks for the training set.
+        for (int o = 0; o < MC_N_OPTIONS; o++)
+            if (config.autotune || o == MC_OPT_REDUCE_MODE || o == MC_OPT_BATCHES) cm.set_option(o, opts[o]);
         const auto t_h2d = std::chrono::steady_clock::now();
         cm.init_parameters(ds);
         const double h2d_s = seconds_since(t_h2d);

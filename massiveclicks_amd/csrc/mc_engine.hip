@@ -1,13 +1,14 @@
 // mc_engine.hip -- kernels and C ABI of the MI355X EM engine.
 //
-// Per EM iteration two kernels run on the model's stream (the held-out
+// Per EM iteration these kernels run on the model's stream (the held-out
 // evaluation is in mc_eval.hip, the gradient path in mc_grad.hip):
 //   em_item_kernel   E-step of one work item per workgroup, per-item
 //                    reduction of the expected counts, in-place M-step of the
 //                    entries the item owns (parallel_em/kernel.cu:42-89 and
-//                    click_models/common.cu:114-192 fused);
-//   em_merge_kernel  M-step of entries merged across items and of the shared
-//                    (rank-indexed) tables.
+//                    click_models/common.cu:114-192 fused); when every item
+//                    has an LDS window, also the M-step of merged entries and
+//                    of the shared (rank-indexed) tables;
+//   em_merge_kernel  otherwise that M-step.
 // theta_t is read from buffer `cur`, theta_{t+1} written to `cur ^ 1`, so the
 // (1,2) reset of the reference (common.cu:71-82, a host fill plus H2D per
 // iteration) disappears: the M-step writes prior + sum directly.
@@ -198,20 +199,40 @@ __device__ __forceinline__ unsigned long long load_acc(const unsigned long long*
 // FP64 bases, threads tid < K; then the accumulators are cleared for the next
 // iteration.  COHERENT: the sums were added during this launch.
 template <bool COHERENT>
-__device__ __forceinline__ void finalize_shared(const KArgs& A, int tid, int nthr) {
+__device__ __forceinline__ void finalize_shared(const KArgs& A, int tid, int nthr, unsigned long long* tot) {
+    for (int j = tid; j < A.kacc; j += nthr) tot[j] = 0ull;
+    __syncthreads();
+    for (int j = tid & (kShStride - 1); j < A.kacc; j += kShStride) {   // one pass: kacc <= kShStride
+        for (int c = tid / kShStride; c < A.sh_parts; c += 8 * (nthr / kShStride)) {
+            unsigned long long v[8];
+#pragma unroll
+            for (int u = 0; u < 8; u++) {
+                const int cu = c + u * (nthr / kShStride);
+                unsigned long long* p = &A.sh_acc[cu * kShStride + j];
+                v[u] = cu < A.sh_parts ? (COHERENT ? load_acc(p) : *p) : 0ull;
+            }
+            unsigned long long w = 0ull;
+#pragma unroll
+            for (int u = 0; u < 8; u++) {
+                const int cu = c + u * (nthr / kShStride);
+                w += v[u];
+                if (v[u] != 0ull) A.sh_acc[cu * kShStride + j] = 0ull;
+            }
+            if (w != 0ull) atomicAdd(&tot[j], w);
+        }
+    }
+    __syncthreads();
     const int k = tid;
     if (k < A.K) {
         const int an = A.sh_acc_map[2 * k], ad = A.sh_acc_map[2 * k + 1];
-        const long long tn = an >= 0 ? (long long)(COHERENT ? load_acc(&A.sh_acc[an]) : A.sh_acc[an]) : 0;
-        const long long td = ad >= 0 ? (long long)(COHERENT ? load_acc(&A.sh_acc[ad]) : A.sh_acc[ad]) : 0;
+        const long long tn = an >= 0 ? (long long)tot[an] : 0;
+        const long long td = ad >= 0 ? (long long)tot[ad] : 0;
         const float num = (float)(A.sh_base[2 * k] + (double)tn * kFixInv);
         const float den = (float)(A.sh_base[2 * k + 1] + (double)td * kFixInv);
         A.sh_num_out[k] = num;
         A.sh_den_out[k] = den;
         A.sh_val_out[k] = clamp_value(num, den);
     }
-    __syncthreads();
-    for (int j = tid; j < A.kacc; j += nthr) A.sh_acc[j] = 0ull;
 }
 
 // M-step of a per-qd entry whose sums several work items added to gacc; the
@@ -231,41 +252,126 @@ __device__ __forceinline__ void finalize_merged_entry(const KArgs& A, int p) {
     }
 }
 
-// Fused M-step of a split query group after a workgroup has added one of
-// its slices: the workgroup that completes the group finalises its entries.
-// Block-uniform call (it.split >= 0); `flag` is a shared int.
+// Counting finished work items in two levels: `c[0]` counts the `parts`
+// counters, c[(1 + p) * kDoneStride] the items p, p + parts, ... of n.
+// done_first counts an item in counter `part` and returns whether that
+// counter is complete; done_last then counts the counter.  One address takes
+// about 13 ns per atomic, so a single counter would serialise the end of a
+// launch of thousands of workgroups.
+__device__ __forceinline__ bool done_first(unsigned* c, unsigned parts, unsigned part, unsigned n) {
+    if (parts == 1u) return true;
+    return atomicAdd(&c[(1u + part) * kDoneStride], 1u) == (n - part + parts - 1u) / parts - 1u;
+}
+__device__ __forceinline__ bool done_last(unsigned* c, unsigned parts, unsigned part, unsigned n) {
+    if (parts > 1u) c[(1u + part) * kDoneStride] = 0u;
+    const bool last = atomicAdd(c, 1u) == (parts > 1u ? min(parts, n) : n) - 1u;
+    if (last) c[0] = 0u;
+    return last;
+}
+
+// Accumulators of the slice's split group in table t (fused M-step).
+__device__ __forceinline__ unsigned long long* split_target(const KArgs& A, const SplitGroup& g, int slice, int t) {
+    return A.split_acc + (int64_t)t * A.n_split_acc + g.acc + (int64_t)(slice & (g.parts - 1)) * (g.hi - g.lo);
+}
+
+// M-step of a split group's entries from the copies of their sums.
 template <int MODEL>
-__device__ __forceinline__ void fused_split_merge(const KArgs& A, const Item& it, int tid, int nthr, int& flag) {
-    wait_memory();
-    __syncthreads();
-    const int4 g = A.split_groups[it.split];
-    if (tid == 0) {
-        flag = atomicAdd(&A.split_done[it.split], 1u) == (unsigned)g.z - 1u;
-        wait_memory();
-    }
-    __syncthreads();
-    if (flag) {
-        wait_memory();
-        for (int p = g.x + tid; p < g.y; p += nthr) finalize_merged_entry<MODEL, true>(A, p);
-        if (tid == 0) A.split_done[it.split] = 0u;
+__device__ __forceinline__ void finalize_split_group(const KArgs& A, const SplitGroup& g, int tid, int nthr) {
+    constexpr int T = Shape<MODEL>::T;
+    const int W = g.hi - g.lo;
+    for (int i = tid; i < W; i += nthr) {
+        const int p = g.lo + i;
+        const int2 oc = A.counts[p];
+#pragma unroll
+        for (int t = 0; t < T; t++) {
+            unsigned long long* a = A.split_acc + (int64_t)t * A.n_split_acc + g.acc + i;
+            const float2 bd = base_den<MODEL>(t, oc);
+            unsigned long long v = 0ull;
+            for (int c = 0; c < g.parts; c++) v += load_acc(a + (int64_t)c * W);
+            for (int c = 0; c < g.parts; c++) a[(int64_t)c * W] = 0ull;
+            const float num = fix_to_float(bd.x, v);
+            A.tab[t].val_out[p] = clamp_value(num, bd.y);
+            if (A.write_num) A.tab[t].num_out[p] = num;
+        }
     }
 }
 
-// Fused M-step of the shared tables: after a workgroup's shared-table sums
-// are in, the last of the launch's n_groups workgroups finalises the tables.
-__device__ __forceinline__ void fused_shared_merge(const KArgs& A, int tid, int nthr, unsigned n_groups, int& flag) {
+// Fused M-step at the end of work item `item`, all of whose sums are on their
+// way: the workgroup that completes its item's split group finalises the
+// group's entries, the last of the iteration's A.n_items items the shared
+// tables.  Block-uniform call; `flag` is a shared int, `tot` shared scratch
+// of kacc sums.
+template <int MODEL>
+__device__ __forceinline__ void fused_merge(const KArgs& A, int item, const Item& it, int tid, int nthr, int& flag,
+                                            unsigned long long* tot) {
+    const int split = it.split, slice = it.flags >> kItemSliceShift;
+    SplitGroup g{};
+    if (split >= 0) g = A.split_groups[split];
     wait_memory();
     __syncthreads();
     if (tid == 0) {
-        flag = atomicAdd(A.grid_done, 1u) == n_groups - 1u;
-        wait_memory();
+        const unsigned n = (unsigned)A.n_items, parts = (unsigned)A.sh_parts, part = (unsigned)item & (parts - 1u);
+        const unsigned gparts = (unsigned)g.parts, gpart = (unsigned)slice & (gparts - 1u);
+        bool a = done_first(A.grid_done, parts, part, n);
+        bool b = split >= 0 && done_first(A.split_done + g.done, gparts, gpart, (unsigned)g.slices);
+        if (a) a = done_last(A.grid_done, parts, part, n);
+        if (b) b = done_last(A.split_done + g.done, gparts, gpart, (unsigned)g.slices);
+        flag = (a ? 1 : 0) | (b ? 2 : 0);
     }
     __syncthreads();
-    if (flag) {
-        wait_memory();
-        finalize_shared<true>(A, tid, nthr);
-        if (tid == 0) *A.grid_done = 0u;
+    const int f = flag;
+    if (f & 2) finalize_split_group<MODEL>(A, g, tid, nthr);
+    if (f & 1) finalize_shared<true>(A, tid, nthr, tot);
+}
+
+// Sums of the lanes' shared-table accumulators over the workgroup, in fixed
+// point (order-independent integer adds), one atomic per accumulator into the
+// workgroup's copy.  `red` holds KACC x NWMAX.
+template <int KACC, int NWMAX>
+__device__ __forceinline__ void add_shared_sums(const KArgs& A, int item, const float (&acc)[55], long long (&red)[KACC][NWMAX],
+                                                int tid, int nthr) {
+    const int wave = tid >> 6, lane = tid & 63, nwave = nthr >> 6;
+#pragma unroll
+    for (int k = 0; k < KACC; k++) {
+        const long long v = wave_sum_last(to_fix(acc[k]));
+        if (lane == 63) red[k][wave] = v;
     }
+    __syncthreads();
+    for (int k = tid; k < KACC; k += nthr) {
+        long long v = 0;
+        for (int w = 0; w < nwave; w++) v += red[k][w];
+        if (v != 0)
+            atomicAdd(&A.sh_acc[(item & (A.sh_parts - 1)) * kShStride + k], (unsigned long long)v);
+    }
+}
+
+// The same for the UBM's examination slots in LDS: the lanes first add their
+// "no earlier click" sums (registers) to their copy of the slots, then eight
+// lanes add up each slot's copies.
+template <int KACC, int NWMAX>
+__device__ __forceinline__ void add_shared_slots(const KArgs& A, int item, const float (&acc)[55], unsigned long long* slots,
+                                                 long long (&red)[KACC][NWMAX], int tid, int nthr) {
+    unsigned long long* mine = slots + (tid & (kUbmCopies - 1));
+#pragma unroll
+    for (int r = 0; r < kL; r++) {
+        const int k = r * (r + 1) / 2 + kL - 1;
+        if (acc[k] != 0.f) atomicAdd(&mine[k * kUbmCopies], (unsigned long long)to_fix(acc[k]));
+    }
+    __syncthreads();
+    for (int q = tid; q < (kUbmSlots + 7) / 8 * 8 * 8; q += nthr) {
+        const int k = q >> 3, c = q & 7;
+        long long v = 0;
+        if (k < kUbmSlots)
+#pragma unroll
+            for (int j = 0; j < kUbmCopies / 8; j++) v += (long long)slots[k * kUbmCopies + c + 8 * j];
+        v += __shfl_xor(v, 1, 64);
+        v += __shfl_xor(v, 2, 64);
+        v += __shfl_xor(v, 4, 64);
+        if (c == 0 && k < kUbmSlots) red[k][0] = v;
+    }
+    __syncthreads();
+    if (tid < kUbmSlots && red[tid][0] != 0)
+        atomicAdd(&A.sh_acc[(item & (A.sh_parts - 1)) * kShStride + tid], (unsigned long long)red[tid][0]);
 }
 
 // Session paths, one kernel instantiation each (each gets its own register
@@ -275,7 +381,13 @@ __device__ __forceinline__ void fused_shared_merge(const KArgs& A, int tid, int 
 enum { kPathLds = 0, kPathGlobal = 1, kPathAtomic = 2, kPathDirect = 3, kPathLdsFloat = 4, kPathPacked = 5 };
 
 // E-step and in-item M-step of one work item (item index item_offset +
-// blockIdx.x).  Dynamic LDS (window path): width x T fixed-point
+// blockIdx.x).  Bound by the VALU on large sets (8M DBN sessions: 380
+// instructions per 64 sessions, about 70 of 82 us) and by the chain of load,
+// session, flush and counter round trips on small ones (32,000 PBM sessions:
+// 5 us of 8, the launch gap included).  At 37-64 VGPRs the packed paths keep
+// 32 wavefronts on a CU, and the hardware hands each freed slot the next
+// item: a persistent form with a fixed item list per workgroup held the next
+// item's window in 77-103 VGPRs and took 87 us on those 8M sessions.  Dynamic LDS (window path): width x T fixed-point
 // accumulators, then width x T staged values of theta_t (both interleaved per
 // entry).  kPathLdsFloat (float-atomic mode) pre-reduces in float LDS
 // accumulators and adds every window entry to global float accumulators,
@@ -290,7 +402,8 @@ __global__ void __launch_bounds__(512) em_item_kernel(KArgs A, int item_offset) 
     __shared__ long long red[KACC][8];
     __shared__ int last_one;
 
-    const Item it = A.items[item_offset + blockIdx.x];
+    const int item = item_offset + (int)blockIdx.x;
+    const Item it = A.items[item];
     const int tid = threadIdx.x;
     const int nthr = blockDim.x;
     const int W = it.width;
@@ -318,22 +431,43 @@ __global__ void __launch_bounds__(512) em_item_kernel(KArgs A, int item_offset) 
     PackedSession r0;
     if (packed) r0 = load_packed(st, it.s0 + tid, it.e1);
     else load_session<VARLEN, win>(st, it.s0 + tid, it.e1, m0, L0, pv0);
-    for (int k = tid; k < K; k += nthr) sh[k] = A.sh_val_in[k];
+    float shv = tid < K ? A.sh_val_in[tid] : 0.f;
     if (win) {
-        for (int i = tid; i < W; i += nthr) {
+        // Three entries' values per lane and pass in flight together, the
+        // first pass's while the accumulators are cleared (1-2 % faster than
+        // one at a time).
+        constexpr int U = 3;
+        for (int i0 = 0; i0 < W; i0 += U * nthr) {
+            float v[U][T];
 #pragma unroll
-            for (int t = 0; t < T; t++) {
-                if (fwin) facc[i * T + t] = 0.f;
-                lval[i * T + t] = A.tab[t].val_in[it.base + i];
+            for (int u = 0; u < U; u++) {
+                if (i0 + u * nthr >= W) break;
+                const int i = min(i0 + u * nthr + tid, W - 1);
+#pragma unroll
+                for (int t = 0; t < T; t++) v[u][t] = A.tab[t].val_in[it.base + i];
+            }
+            if (i0 == 0) {
+                if (fwin) {
+                    for (int i = tid; i < W * T; i += nthr) facc[i] = 0.f;
+                } else {
+                    for (int i = tid; i < WS; i += nthr)
+#pragma unroll
+                        for (int t = 0; t < T; t++) lacc[aw.slot(t, i)] = 0ull;
+                }
+                if (lslots)
+                    for (int i = tid; i < kUbmSlots * kUbmCopies; i += nthr) slots[i] = 0ull;
+            }
+#pragma unroll
+            for (int u = 0; u < U; u++) {
+                const int i = i0 + u * nthr + tid;
+                if (i0 + u * nthr >= W) break;
+#pragma unroll
+                for (int t = 0; t < T; t++)
+                    if (i < W) lval[i * T + t] = v[u][t];
             }
         }
-        if (!fwin)
-            for (int i = tid; i < WS; i += nthr)
-#pragma unroll
-                for (int t = 0; t < T; t++) lacc[aw.slot(t, i)] = 0ull;
     }
-    if (lslots)
-        for (int i = tid; i < kUbmSlots * kUbmCopies; i += nthr) slots[i] = 0ull;
+    if (tid < K) sh[tid] = shv;
     __syncthreads();
 
     float acc[55];
@@ -360,22 +494,9 @@ __global__ void __launch_bounds__(512) em_item_kernel(KArgs A, int item_offset) 
         run_item<MODEL, VARLEN, false>(st, it, gsrc, em, sh, acc, m0, L0, pv0);
     }
 
-    // Shared tables: fixed point, wave sums, across waves, one atomic per
-    // accumulator and work item (integer adds: order-independent).
-    const int wave = tid >> 6, lane = tid & 63, nwave = nthr >> 6;
-#pragma unroll
-    for (int k = 0; k < KACC; k++) {
-        long long v = wave_sum(to_fix(acc[k]));
-        if (lane == 0) red[k][wave] = v;
-    }
-    __syncthreads();
-    for (int k = tid; k < KACC; k += nthr) {
-        long long v = 0;
-        for (int w = 0; w < nwave; w++) v += red[k][w];
-        if (lslots)
-            for (int c = 0; c < kUbmCopies; c++) v += (long long)slots[k * kUbmCopies + c];
-        if (v != 0) atomicAdd(&A.sh_acc[k], (unsigned long long)v);
-    }
+    // Shared tables (also the barrier before the window is flushed).
+    if constexpr (lslots) add_shared_slots<KACC>(A, item, acc, slots, red, tid, nthr);
+    else add_shared_sums<KACC>(A, item, acc, red, tid, nthr);
 
     if (fwin) {
         for (int i = tid; i < W; i += nthr) {
@@ -388,8 +509,14 @@ __global__ void __launch_bounds__(512) em_item_kernel(KArgs A, int item_offset) 
     }
     // Flush the LDS window, four entries per thread per pass with the
     // constant loads issued together.
-    if (win && !fwin) {
+    if (fixwin) {
         const bool interior = (it.flags & kItemInterior) != 0;
+        unsigned long long* sink[T];
+#pragma unroll
+        for (int t = 0; t < T; t++)
+            sink[t] = (A.fuse_merge && it.split >= 0)
+                          ? split_target(A, A.split_groups[it.split], it.flags >> kItemSliceShift, t)
+                          : A.tab[t].gacc + it.base;
         for (int i0 = 0; i0 < W; i0 += 4 * nthr) {
             uint32_t pk[4];
 #pragma unroll
@@ -412,214 +539,13 @@ __global__ void __launch_bounds__(512) em_item_kernel(KArgs A, int item_offset) 
                         A.tab[t].val_out[p] = clamp_value(num, bd.y);
                         if (A.write_num) A.tab[t].num_out[p] = num;
                     } else if (v != 0ull) {
-                        atomicAdd(&A.tab[t].gacc[p], v);
+                        atomicAdd(&sink[t][i], v);
                     }
                 }
             }
         }
     }
-    // Fused M-step (the launch is the iteration's only E-step launch): split
-    // groups, then the shared tables, as in the persistent kernel.
-    if (A.fuse_merge) {
-        if (it.split >= 0) fused_split_merge<MODEL>(A, it, tid, nthr, last_one);
-        fused_shared_merge(A, tid, nthr, gridDim.x, last_one);
-    }
-}
-
-// Persistent form of the window path over items [first, first + n_win), all
-// packed (PACKED) or all rank-major: workgroup b of G resident ones
-// processes one window item per round, item kG + b in even rounds k and
-// kG + G - 1 - b in odd ones.  Items are ordered largest first, so this
-// back-and-forth order pairs the larger items of one round with the smaller
-// of the next, while the items of a round stay adjacent in memory; a fixed
-// assignment keeps the per-lane float sums, and so the results, identical
-// from run to run.
-// While item k is processed, the window values of the workgroup's next item
-// and its first session are in flight (registers), and the constants of
-// item k's entries arrive during its session loop, so the round trips of
-// staging and flushing overlap with the E-step and the flush.  The shared-table counts stay
-// in registers across items and are reduced once per workgroup.  Requires
-// blockDim.x == 256 and width <= 256 * PER.
-// Waves per SIMD the persistent kernel asks the compiler to fit: ten-rank DBN
-// goes from 4 waves (108 VGPRs) to 5 (89-95 VGPRs, no spills), 1-3 %
-// faster (at 6, 80 VGPRs with spills, it is 8 % slower and its 1280-entry
-// window's LDS allows only 5 workgroups per CU anyway); ten-rank CCM over
-// packed sessions runs 6 (80 VGPRs, 5 dwords spilled; one per-qd table, so
-// 6 windows fit), 2-3 % faster than 5 (its rank-major form would spill 15
-// dwords and keeps 5); the uneven-length UBM kernel goes from 2 waves (181 VGPRs)
-// to 3 (168 VGPRs, 4 dwords spilled), 22 % faster.  Ten-rank PBM fits 7
-// without a hint (the host caps it at 6 per CU: 7 measured slower), and
-// ten-rank UBM fits 6 (79 VGPRs) but its window plus examination slots
-// allow 5 workgroups per CU.
-template <int MODEL, bool VARLEN, bool PACKED>
-struct PersistWaves {
-    static constexpr int value = (!VARLEN && MODEL == kDBN)   ? 5
-                                 : (!VARLEN && MODEL == kCCM) ? (PACKED ? 6 : 5)
-                                 : (VARLEN && MODEL == kUBM)  ? 3
-                                                              : 1;
-};
-
-template <int MODEL, bool VARLEN, int PER, bool PACKED>
-__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(PersistWaves<MODEL, VARLEN, PACKED>::value)))
-em_window_persistent_kernel(KArgs A, int first, int n_win) {
-    constexpr int T = Shape<MODEL>::T;
-    constexpr int K = Shape<MODEL>::K;
-    constexpr int KACC = Shape<MODEL>::KACC;
-    constexpr int NT = 256;
-    extern __shared__ unsigned long long lds[];
-    __shared__ float sh[K < 64 ? 64 : K];
-    __shared__ long long red[KACC][4];
-    __shared__ int last_one;
-
-    const int tid = threadIdx.x;
-    const int Wmax = A.max_width;
-    unsigned long long* lacc = lds;
-    float* lval = (float*)(lds + T * Wmax);
-    // UBM examination slots in LDS after the window, kept across items.
-    constexpr bool lslots = MODEL == kUBM;
-    unsigned long long* slots = lds + ((size_t)T * Wmax * 12 + 7) / 8;
-    if (lslots)
-        for (int i = tid; i < kUbmSlots * kUbmCopies; i += NT) slots[i] = 0ull;
-    const Stream st = make_stream(A);
-    for (int k = tid; k < K; k += NT) sh[k] = A.sh_val_in[k];
-
-    const int G = (int)gridDim.x;
-    auto item_of_round = [&](int k) { return k * G + ((k & 1) ? G - 1 - (int)blockIdx.x : (int)blockIdx.x); };
-    int round = 0;
-    int cur = item_of_round(0);
-    Item it = cur < n_win ? A.items[first + cur] : Item{};
-
-    // Window values of the current item, and its first session.
-    float wv[PER][T];
-#pragma unroll
-    for (int u = 0; u < PER; u++) {
-        const int i = u * NT + tid;
-#pragma unroll
-        for (int t = 0; t < T; t++) wv[u][t] = (i < it.width) ? A.tab[t].val_in[it.base + i] : 0.f;
-    }
-    uint32_t m0 = 0;
-    int L0 = 0;
-    int pv0[kL];
-    PackedSession r0;
-    if (PACKED) r0 = load_packed(st, it.s0 + tid, it.e1);
-    else load_session<VARLEN, true>(st, it.s0 + tid, it.e1, m0, L0, pv0);
-
-    float acc[55];
-#pragma unroll
-    for (int k = 0; k < 55; k++) acc[k] = 0.f;
-
-    while (cur < n_win) {
-        const int W = it.width;
-        const AccWindow<T> aw{lacc, Wmax, acc_copies_log2(W, Wmax)};
-        const int WS = W << aw.rsh;
-        // Stage the window, take the next item.
-#pragma unroll
-        for (int u = 0; u < PER; u++) {
-            const int i = u * NT + tid;
-            if (i < W) {
-#pragma unroll
-                for (int t = 0; t < T; t++) lval[i * T + t] = wv[u][t];
-            }
-            if (i < WS) {
-#pragma unroll
-                for (int t = 0; t < T; t++) lacc[aw.slot(t, i)] = 0ull;
-            }
-        }
-        __syncthreads();
-        const int nxt = item_of_round(round + 1);
-        const Item itn = nxt < n_win ? A.items[first + nxt] : Item{};
-        // In flight during the session loop: next window values, this
-        // window's counts.
-        // Ten-rank kernels load the next window after the session loop
-        // instead (its latency then overlaps the flush), which frees the
-        // window registers during the loop: fewer spills at 5 waves per SIMD,
-        // 1-3 % faster; the uneven-length kernels measured 1-3 % slower so.
-        constexpr bool LATE_WINDOW = !VARLEN;
-        uint32_t cnt[PER];
-#pragma unroll
-        for (int u = 0; u < PER; u++) {
-            const int i = u * NT + tid;
-            if (!LATE_WINDOW) {
-#pragma unroll
-                for (int t = 0; t < T; t++) wv[u][t] = (i < itn.width) ? A.tab[t].val_in[itn.base + i] : 0.f;
-            }
-            cnt[u] = (i < W) ? A.counts16[it.base + i] : 0u;
-        }
-        {
-            EmitLds<T> em{aw, tid & ((1 << aw.rsh) - 1), slots + (tid & (kUbmCopies - 1))};
-            const SrcLds<T> lsrc{lval};
-            if (PACKED) run_item_packed<MODEL, VARLEN>(st, it, lsrc, em, sh, acc, r0);
-            else run_item<MODEL, VARLEN, true>(st, it, lsrc, em, sh, acc, m0, L0, pv0);
-        }
-        const bool interior = (it.flags & kItemInterior) != 0;
-        // Full counts of the entries with 255 or more occurrences, loaded
-        // before the prefetches below and without a branch (lanes without
-        // such an entry read the item's first entry, a line the wave
-        // shares): a conditional load per entry made the flush wait, entry
-        // by entry, for everything in flight, the prefetches and the
-        // previous entry's stores included (PBM and UBM 5 % slower).
-        int2 full[PER];
-#pragma unroll
-        for (int u = 0; u < PER; u++) {
-            const int i = u * NT + tid;
-            full[u] = A.counts[cnt[u] == kCountsEscape ? it.base + i : it.base];
-        }
-        if (LATE_WINDOW) {
-#pragma unroll
-            for (int u = 0; u < PER; u++) {
-                const int i = u * NT + tid;
-#pragma unroll
-                for (int t = 0; t < T; t++) wv[u][t] = (i < itn.width) ? A.tab[t].val_in[itn.base + i] : 0.f;
-            }
-        }
-        // First session of the next item goes out before the flush.
-        if (PACKED) r0 = load_packed(st, itn.s0 + tid, itn.e1);
-        else load_session<VARLEN, true>(st, itn.s0 + tid, itn.e1, m0, L0, pv0);
-        __syncthreads();
-#pragma unroll
-        for (int u = 0; u < PER; u++) {
-            const int i = u * NT + tid;
-            if (i >= W) continue;
-            const int p = it.base + i;
-            const int2 ocu = interior ? unpack_counts(cnt[u], full[u]) : make_int2(0, 0);
-#pragma unroll
-            for (int t = 0; t < T; t++) {
-                const unsigned long long v = aw.sum(t, i);
-                if (interior) {
-                    const float2 bd = base_den<MODEL>(t, ocu);
-                    const float num = fix_to_float(bd.x, v);
-                    A.tab[t].val_out[p] = clamp_value(num, bd.y);
-                    if (A.write_num) A.tab[t].num_out[p] = num;
-                } else if (v != 0ull) {
-                    atomicAdd(&A.tab[t].gacc[p], v);
-                }
-            }
-        }
-        // Fused M-step of a split query group: the workgroup that adds the
-        // group's last slice finalises the group's entries.
-        if (A.fuse_merge && it.split >= 0) fused_split_merge<MODEL>(A, it, tid, NT, last_one);
-        __syncthreads();
-        round++;
-        cur = nxt;
-        it = itn;
-    }
-
-    // Shared tables: one reduction and one atomic per accumulator per workgroup.
-    const int wave = tid >> 6, lane = tid & 63;
-#pragma unroll
-    for (int k = 0; k < KACC; k++) {
-        long long v = wave_sum(to_fix(acc[k]));
-        if (lane == 0) red[k][wave] = v;
-    }
-    __syncthreads();
-    for (int k = tid; k < KACC; k += NT) {
-        long long v = red[k][0] + red[k][1] + red[k][2] + red[k][3];
-        if (lslots)
-            for (int c = 0; c < kUbmCopies; c++) v += (long long)slots[k * kUbmCopies + c];
-        if (v != 0) atomicAdd(&A.sh_acc[k], (unsigned long long)v);
-    }
-    // Fused M-step of the shared tables: the last workgroup to finish.
-    if (A.fuse_merge) fused_shared_merge(A, tid, NT, (unsigned)G, last_one);
+    if (A.fuse_merge) fused_merge<MODEL>(A, item, it, tid, nthr, last_one, (unsigned long long*)red);
 }
 
 // Merge kernel: block 0 finalises the shared tables, the other blocks
@@ -630,7 +556,8 @@ __global__ void __launch_bounds__(256) em_merge_kernel(KArgs A) {
     constexpr int T = Shape<MODEL>::T;
     const int tid = threadIdx.x;
     if (blockIdx.x == 0) {
-        finalize_shared<false>(A, tid, (int)blockDim.x);
+        __shared__ unsigned long long tot[kShStride];
+        finalize_shared<false>(A, tid, (int)blockDim.x, tot);
         return;
     }
     const int64_t i = (int64_t)(blockIdx.x - 1) * blockDim.x + tid;
@@ -758,57 +685,24 @@ KArgs make_args(mc_model* m, int cur, int write_num) {
     A.sh_den_out = m->d_sh_den[cur ^ 1];
     A.fuse_merge = m->fuse ? 1 : 0;
     A.split_groups = m->d_split_groups;
+    A.split_acc = m->d_split_acc;
+    A.n_split_acc = m->n_split_acc;
     A.split_done = m->d_split_done;
     A.grid_done = m->d_grid_done;
+    A.sh_parts = m->sh_parts;
     return A;
 }
 
+// `width`: the launch's window entries (LDS), 0 for items without a window.
 template <int MODEL, int PATH>
-void launch_path(mc_model* m, const KArgs& A, int first, int count, size_t lds) {
+void launch_path(mc_model* m, KArgs A, int first, int count, int width) {
     if (count <= 0) return;
+    A.max_width = width;
+    const size_t lds = width ? window_lds_bytes(m->type, m->reduce_mode, width) : 0;
     if (m->varlen)
         hipLaunchKernelGGL((em_item_kernel<MODEL, true, PATH>), dim3(count), dim3(m->block), lds, m->stream, A, first);
     else
         hipLaunchKernelGGL((em_item_kernel<MODEL, false, PATH>), dim3(count), dim3(m->block), lds, m->stream, A, first);
-}
-
-// Window width covered by the persistent kernel's register staging.
-constexpr int kPersistPer = 5;
-
-// Resident workgroups per CU of the model's persistent window kernel.
-template <int MODEL, bool PACKED>
-hipError_t persistent_occupancy_of(const mc_model* m, int* per_cu) {
-    return m->varlen
-               ? hipOccupancyMaxActiveBlocksPerMultiprocessor(
-                     per_cu, em_window_persistent_kernel<MODEL, true, kPersistPer, PACKED>, 256, m->lds_bytes)
-               : hipOccupancyMaxActiveBlocksPerMultiprocessor(
-                     per_cu, em_window_persistent_kernel<MODEL, false, kPersistPer, PACKED>, 256, m->lds_bytes);
-}
-
-template <bool PACKED>
-hipError_t persistent_occupancy_pk(const mc_model* m, int* per_cu) {
-    switch (m->type) {
-        case MC_PBM: return persistent_occupancy_of<kPBM, PACKED>(m, per_cu);
-        case MC_UBM: return persistent_occupancy_of<kUBM, PACKED>(m, per_cu);
-        case MC_DBN: return persistent_occupancy_of<kDBN, PACKED>(m, per_cu);
-        default: return persistent_occupancy_of<kCCM, PACKED>(m, per_cu);
-    }
-}
-
-hipError_t persistent_occupancy(const mc_model* m, bool packed, int* per_cu) {
-    return packed ? persistent_occupancy_pk<true>(m, per_cu) : persistent_occupancy_pk<false>(m, per_cu);
-}
-
-template <int MODEL, bool PACKED>
-void launch_persistent(mc_model* m, const KArgs& A, int first, int count) {
-    if (count <= 0) return;
-    const dim3 grid((unsigned)std::min(count, m->persist_grid[PACKED]));
-    if (m->varlen)
-        hipLaunchKernelGGL((em_window_persistent_kernel<MODEL, true, kPersistPer, PACKED>), grid, dim3(256),
-                           m->lds_bytes, m->stream, A, first, count);
-    else
-        hipLaunchKernelGGL((em_window_persistent_kernel<MODEL, false, kPersistPer, PACKED>), grid, dim3(256),
-                           m->lds_bytes, m->stream, A, first, count);
 }
 
 template <int MODEL>
@@ -816,17 +710,11 @@ void launch_item(mc_model* m, const KArgs& A) {
     if (m->reduce_mode == MC_REDUCE_ATOMIC) {
         // LDS pre-reduction of window items, then float atomics; items
         // without a window add straight to the global accumulators.
-        launch_path<MODEL, kPathLdsFloat>(m, A, 0, m->n_win_items, m->lds_bytes);
+        launch_path<MODEL, kPathLdsFloat>(m, A, 0, m->n_win_items, m->max_width);
         launch_path<MODEL, kPathAtomic>(m, A, m->n_win_items, m->n_glob_items, 0);
     } else {
-        const int n_pk = m->n_pk_items, n_rm = m->n_win_items - m->n_pk_items;
-        if (m->persistent) {
-            launch_persistent<MODEL, true>(m, A, 0, n_pk);
-            launch_persistent<MODEL, false>(m, A, n_pk, n_rm);
-        } else {
-            launch_path<MODEL, kPathPacked>(m, A, 0, n_pk, m->lds_bytes);
-            launch_path<MODEL, kPathLds>(m, A, n_pk, n_rm, m->lds_bytes);
-        }
+        launch_path<MODEL, kPathPacked>(m, A, 0, m->n_pk_items, m->max_width);
+        launch_path<MODEL, kPathLds>(m, A, m->n_pk_items, m->n_win_items - m->n_pk_items, m->max_width);
         launch_path<MODEL, kPathGlobal>(m, A, m->n_win_items, m->n_glob_items, 0);
         launch_path<MODEL, kPathDirect>(m, A, m->n_win_items + m->n_glob_items, m->n_dir_items, 0);
     }
@@ -845,7 +733,7 @@ mc_status launch_estep(mc_model* m, int cur, int write_num) {
 }
 
 mc_status launch_mstep(mc_model* m, int cur, int write_num) {
-    if (m->fuse) return MC_OK;   // done by the persistent kernel
+    if (m->fuse) return MC_OK;   // done by the E-step launches
     KArgs A = make_args(m, cur, write_num);
     int64_t n_entries = m->reduce_mode == MC_REDUCE_ATOMIC ? m->n_qd : m->n_shared;
     unsigned grid = (unsigned)(1 + (n_entries + 255) / 256);
@@ -938,6 +826,7 @@ mc_status mc_model_set_option(mc_model* m, int option, int64_t value) {
         case MC_OPT_ITEM_SESSIONS:
             MC_REQUIRE(value >= 64 && value <= (1 << 20), "item sessions out of range [64, 2^20]");
             m->item_sessions = (int)value;
+            m->item_sessions_set = true;
             break;
         case MC_OPT_ITEM_WINDOW:
             MC_REQUIRE(value >= 0 && value <= 16384, "item window out of range [0, 16384]");
@@ -950,8 +839,7 @@ mc_status mc_model_set_option(mc_model* m, int option, int64_t value) {
             m->direct = value != 0;
             break;
         case MC_OPT_PERSISTENT:
-            m->persistent = value != 0;
-            break;
+            break;   // no effect
         case MC_OPT_PACKED:
             m->packed = value != 0;
             break;
@@ -968,6 +856,7 @@ mc_status mc_model_set_option(mc_model* m, int option, int64_t value) {
         case MC_OPT_BLOCK:
             MC_REQUIRE(value == 64 || value == 128 || value == 256 || value == 512, "block must be 64/128/256/512");
             m->block = (int)value;
+            m->block_set = true;
             break;
         default:
             set_error("unknown option");
@@ -998,7 +887,6 @@ mc_status mc_init_parameters(mc_model* m, int64_t n, const int32_t* query, const
         set_error("out of host memory while planning the device layout");
         return MC_ERR_OOM;
     }
-    const int max_width = m->max_width;
     const std::vector<Item>& items = h.items;
     const std::vector<int32_t>& shared_idx = h.shared_idx;
     const std::vector<int32_t>& lists = h.lists;
@@ -1014,35 +902,18 @@ mc_status mc_init_parameters(mc_model* m, int64_t n, const int32_t* query, const
         // workgroup's LDS.
         int max_lds = 0;
         MC_HIP(hipDeviceGetAttribute(&max_lds, hipDeviceAttributeMaxSharedMemoryPerBlock, m->device));
-        MC_REQUIRE(m->lds_bytes + 4096 <= (size_t)max_lds,
-                   "item window too large for this device's LDS (" + std::to_string(max_width) + " entries need " +
-                       std::to_string(m->lds_bytes) + " bytes, at most " + std::to_string(max_lds) +
+        const size_t lds = window_lds_bytes(m->type, m->reduce_mode, m->max_width);
+        MC_REQUIRE(lds + 4096 <= (size_t)max_lds,
+                   "item window too large for this device's LDS (" + std::to_string(m->max_width) + " entries need " +
+                       std::to_string(lds) + " bytes, at most " + std::to_string(max_lds) +
                        " per workgroup): use a smaller MC_OPT_ITEM_WINDOW");
     }
 
-    // Persistent window kernel: 256-thread workgroups, windows staged through
-    // registers (width <= 256 * kPersistPer), one workgroup per resident slot.
-    m->persistent = m->persistent && m->block == 256 && max_width <= 256 * kPersistPer;
-    // The M-step runs inside the E-step kernel when that kernel is the
-    // iteration's only launch (every work item a window item, all of one
-    // session format) in the segmented mode: the persistent kernel or the
-    // one-workgroup-per-item kernel.
-    m->fuse = m->fused_merge && m->reduce_mode == MC_REDUCE_SEGMENTED && m->n_win_items > 0 &&
-              m->n_glob_items == 0 && m->n_dir_items == 0 &&
-              (m->n_pk_items == 0 || m->n_pk_items == m->n_win_items);
-    if (m->persistent && m->n_win_items > 0) {
-        int n_cu = 0;
-        MC_HIP(hipDeviceGetAttribute(&n_cu, hipDeviceAttributeMultiprocessorCount, m->device));
-        for (int pk = 0; pk < 2; pk++) {
-            int per_cu = 0;
-            MC_HIP(persistent_occupancy(m, pk != 0, &per_cu));
-            // At most 6 workgroups per CU: the ten-rank PBM kernel (71 VGPRs)
-            // fits 7, which measured 4 % slower (0.080 -> 0.084 ms per
-            // iteration over 8M sessions) with one more window staged per CU.
-            m->persist_grid[pk] = std::max(1, std::min(per_cu, 6) * n_cu);
-        }
-    }
-
+    // The M-step runs inside the E-step launches when every work item is a
+    // window item of the segmented mode.
+    m->fuse = m->fused_merge && m->reduce_mode == MC_REDUCE_SEGMENTED && m->n_win_items == m->n_items;
+    m->sh_parts = 1;
+    while (m->sh_parts < kMaxShParts && m->sh_parts * 32 < m->n_items) m->sh_parts *= 2;
     MC_TRY(dalloc(m, &m->d_packed, std::max<size_t>(h.packed.size() * 4, 16)));
     MC_TRY(dalloc(m, &m->d_pidx16, std::max<size_t>(h_pidx16.size() * 2, 4)));
     MC_TRY(dalloc(m, &m->d_pidx, std::max<size_t>(h_pidx.size() * 4, 4)));
@@ -1050,9 +921,26 @@ mc_status mc_init_parameters(mc_model* m, int64_t n, const int32_t* query, const
     if (m->varlen) MC_TRY(dalloc(m, &m->d_len, h_len.size()));
     MC_TRY(dalloc(m, &m->d_items, items.size() * sizeof(Item)));
     MC_TRY(dalloc(m, &m->d_shared_idx, shared_idx.size() * 4));
-    MC_TRY(dalloc(m, &m->d_split_groups, std::max<size_t>(h.split_groups.size(), 1) * sizeof(int4)));
-    MC_TRY(dalloc(m, &m->d_split_done, std::max<size_t>(h.split_groups.size(), 1) * 4));
-    MC_TRY(dalloc(m, &m->d_grid_done, 4));
+    // Copies of the split groups' sums and counters: one copy per eight
+    // slices, at most 16 and 4096 accumulators a group.
+    int64_t n_split_done = 0;
+    m->n_split_acc = 0;
+    if (m->fuse)
+        for (SplitGroup& g : h.split_groups) {
+            g.parts = 1;
+            while (g.parts < 16 && g.parts * 16 <= g.slices && (int64_t)g.parts * 2 * (g.hi - g.lo) <= 4096) g.parts *= 2;
+            MC_REQUIRE(m->n_split_acc < (1 << 30) && n_split_done < (1 << 30), "internal: split group sums");
+            g.acc = (int32_t)m->n_split_acc;
+            g.done = (int32_t)n_split_done;
+            m->n_split_acc += (int64_t)g.parts * (g.hi - g.lo);
+            n_split_done += (int64_t)(1 + g.parts) * kDoneStride;
+        }
+    const size_t split_acc_bytes = (size_t)std::max<int64_t>(m->n_split_acc, 1) * T * 8;
+    const size_t split_done_bytes = (size_t)std::max<int64_t>(n_split_done, 1) * 4;
+    MC_TRY(dalloc(m, &m->d_split_groups, std::max<size_t>(h.split_groups.size(), 1) * sizeof(SplitGroup)));
+    MC_TRY(dalloc(m, &m->d_split_acc, split_acc_bytes));
+    MC_TRY(dalloc(m, &m->d_split_done, split_done_bytes));
+    MC_TRY(dalloc(m, &m->d_grid_done, (size_t)(1 + m->sh_parts) * kDoneStride * 4));
     MC_TRY(dalloc(m, &m->d_lists, lists.size() * 4));
     for (int t = 0; t < T; t++) {
         for (int b = 0; b < 2; b++) {
@@ -1070,7 +958,7 @@ mc_status mc_init_parameters(mc_model* m, int64_t n, const int32_t* query, const
     MC_TRY(dalloc(m, &m->d_counts16, (size_t)n_qd * 2));
     MC_TRY(dalloc(m, &m->d_sh_base, sh_base.size() * 8));
     MC_TRY(dalloc(m, &m->d_sh_acc_map, sh_map.size() * 4));
-    MC_TRY(dalloc(m, &m->d_sh_acc, (size_t)KACC * 8));
+    MC_TRY(dalloc(m, &m->d_sh_acc, (size_t)m->sh_parts * kShStride * 8));
 
     if (!h.packed.empty())
         MC_HIP(hipMemcpyAsync(m->d_packed, h.packed.data(), h.packed.size() * 4, hipMemcpyHostToDevice, m->stream));
@@ -1086,10 +974,11 @@ mc_status mc_init_parameters(mc_model* m, int64_t n, const int32_t* query, const
         MC_HIP(hipMemcpyAsync(m->d_shared_idx, shared_idx.data(), shared_idx.size() * 4, hipMemcpyHostToDevice,
                               m->stream));
     if (!h.split_groups.empty())
-        MC_HIP(hipMemcpyAsync(m->d_split_groups, h.split_groups.data(), h.split_groups.size() * sizeof(int4),
+        MC_HIP(hipMemcpyAsync(m->d_split_groups, h.split_groups.data(), h.split_groups.size() * sizeof(SplitGroup),
                               hipMemcpyHostToDevice, m->stream));
-    MC_HIP(hipMemsetAsync(m->d_split_done, 0, std::max<size_t>(h.split_groups.size(), 1) * 4, m->stream));
-    MC_HIP(hipMemsetAsync(m->d_grid_done, 0, 4, m->stream));
+    MC_HIP(hipMemsetAsync(m->d_split_acc, 0, split_acc_bytes, m->stream));
+    MC_HIP(hipMemsetAsync(m->d_split_done, 0, split_done_bytes, m->stream));
+    MC_HIP(hipMemsetAsync(m->d_grid_done, 0, (size_t)(1 + m->sh_parts) * kDoneStride * 4, m->stream));
     if (!lists.empty())
         MC_HIP(hipMemcpyAsync(m->d_lists, lists.data(), lists.size() * 4, hipMemcpyHostToDevice, m->stream));
     MC_HIP(hipMemcpyAsync(m->d_counts, counts.data(), counts.size() * 8, hipMemcpyHostToDevice, m->stream));
@@ -1100,7 +989,7 @@ mc_status mc_init_parameters(mc_model* m, int64_t n, const int32_t* query, const
     MC_HIP(hipMemcpyAsync(m->d_counts16, counts16.data(), counts16.size() * 2, hipMemcpyHostToDevice, m->stream));
     MC_HIP(hipMemcpyAsync(m->d_sh_base, sh_base.data(), sh_base.size() * 8, hipMemcpyHostToDevice, m->stream));
     MC_HIP(hipMemcpyAsync(m->d_sh_acc_map, sh_map.data(), sh_map.size() * 4, hipMemcpyHostToDevice, m->stream));
-    MC_HIP(hipMemsetAsync(m->d_sh_acc, 0, (size_t)KACC * 8, m->stream));
+    MC_HIP(hipMemsetAsync(m->d_sh_acc, 0, (size_t)m->sh_parts * kShStride * 8, m->stream));
     for (int t = 0; t < T; t++) {
         MC_HIP(hipMemsetAsync(m->d_gacc[t], 0, (size_t)n_qd * 8, m->stream));
         for (int b = 0; b < 2; b++) {

@@ -703,6 +703,9 @@ GArgs make_gargs(mc_model* m, int batch) {
     return G;
 }
 
+// Accumulators and staged values of the widest window.
+size_t grad_lds_bytes(const mc_model* m) { return (size_t)m->max_width * m->T * 12; }
+
 template <int MODEL, bool WIN, bool ADAM, int NT>
 void launch_items(mc_model* m, const GArgs& G, int64_t count, int64_t off, size_t lds) {
     if (m->varlen)
@@ -724,8 +727,8 @@ void launch_grad_t(mc_model* m, const GArgs& G0, int batch) {
     // Few items (a small minibatch): 1024 lanes per item to fill the chip.
     const bool wide = nw + ng < 4 * (int64_t)m->n_cu;
     if (nw > 0) {
-        if (wide) launch_items<MODEL, true, ADAM, 1024>(m, G, nw, m->win_off[b], m->lds_bytes);
-        else launch_items<MODEL, true, ADAM, 256>(m, G, nw, m->win_off[b], m->lds_bytes);
+        if (wide) launch_items<MODEL, true, ADAM, 1024>(m, G, nw, m->win_off[b], grad_lds_bytes(m));
+        else launch_items<MODEL, true, ADAM, 256>(m, G, nw, m->win_off[b], grad_lds_bytes(m));
     }
     if (ng > 0) {
         if (wide) launch_items<MODEL, false, ADAM, 1024>(m, G, ng, m->glob_off[b], 0);
@@ -778,8 +781,8 @@ void launch_fused_step_t(mc_model* m, int b) {
         const int64_t nw = m->win_cnt[bi], ng = m->glob_cnt[bi];
         const bool wide = nw + ng < 4 * (int64_t)m->n_cu;
         if (nw > 0) {
-            if (wide) launch_items<MODEL, true, true, 1024>(m, G, nw, m->win_off[bi], m->lds_bytes);
-            else launch_items<MODEL, true, true, 256>(m, G, nw, m->win_off[bi], m->lds_bytes);
+            if (wide) launch_items<MODEL, true, true, 1024>(m, G, nw, m->win_off[bi], grad_lds_bytes(m));
+            else launch_items<MODEL, true, true, 256>(m, G, nw, m->win_off[bi], grad_lds_bytes(m));
         }
         if (ng > 0) {
             // A second launch of the same step: the finalisation is done and

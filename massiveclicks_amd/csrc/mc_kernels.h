@@ -37,6 +37,7 @@ enum { kPBM = 0, kCCM = 1, kDBN = 2, kUBM = 3 };
 // 16-byte records (every session's indices lie within 256 consecutive
 // window entries).
 enum { kItemInterior = 1, kItemDirect = 2, kItemPacked = 4 };
+constexpr int kItemSliceShift = 8;   // flags >> 8: slice number of a split group's item
 
 struct Item {
     int32_t s0, s1;     // session range [s0, s1) in device order
@@ -52,6 +53,18 @@ struct Item {
                         // path alone
     int32_t split;      // slices of one query group: the group's index in
                         // KArgs::split_groups, else -1
+};
+
+// A query group whose sessions are split over several window items.  Slice k
+// adds its sums to copy k % parts of the group's accumulators and counts in
+// counter k % parts, so that the hundreds of slices of a heavy query don't
+// queue on the addresses of its few entries.
+struct SplitGroup {
+    int32_t lo, hi;       // entries
+    int32_t slices;
+    int32_t parts;        // power of two
+    int32_t acc;          // first accumulator (of parts x (hi - lo)) in KArgs::split_acc
+    int32_t done;         // first counter in KArgs::split_done
 };
 
 struct TableArgs {
@@ -84,7 +97,7 @@ struct KArgs {
     const int2* counts;       // per qd entry: (occurrences, clicked occurrences) in training
     const uint16_t* counts16; // the same packed as o | c << 8 when o < 255, else kCountsEscape
     const float* sh_val_in;   // shared table values of theta_t
-    unsigned long long* sh_acc;   // [kacc] fixed-point accumulators of the shared tables
+    unsigned long long* sh_acc;   // [sh_parts][kShStride] fixed-point accumulators of the shared tables
     int32_t max_width;            // largest item window (LDS sizing)
     // merge kernel
     const int32_t* shared_idx;   // entries merged across items
@@ -100,14 +113,27 @@ struct KArgs {
     float* sh_val_out;
     float* sh_num_out;
     float* sh_den_out;
-    // M-step inside the persistent kernel (fuse_merge): the last slice of a
+    // M-step inside the E-step launches (fuse_merge): the last slice of a
     // split query group to finish finalises the group's entries, the last
-    // workgroup the shared tables; counters return to 0 for the next launch.
+    // item the shared tables; counters return to 0 for the next iteration.
     int32_t fuse_merge;
-    const int4* split_groups;     // per split group: first entry, end entry, slices
-    unsigned* split_done;         // per split group: slices finished
-    unsigned* grid_done;          // workgroups finished
+    const SplitGroup* split_groups;
+    unsigned long long* split_acc;   // [T][n_split_acc] sums of the split groups' slices
+    int64_t n_split_acc;
+    unsigned* split_done;         // slices finished, per group [parts + 1] counters kDoneStride apart
+    unsigned* grid_done;          // workgroups finished: [sh_parts + 1] counters kDoneStride apart
+    int32_t sh_parts;             // copies of the shared-table sums and of the counter (power of two)
 };
+
+// The shared-table sums and the count of finished workgroups are kept in
+// `sh_parts` copies, one cache line or more apart: work item i uses copy
+// i % sh_parts, so that thousands of workgroups don't queue on one address.
+// One per XCD (8): 312k UBM sessions in 395 items 17.8 us per iteration with
+// one copy, 13.3 with 8, 14.5 with 32 (the last workgroup reads them all); 8M
+// DBN sessions in 6,147 items 113 us with one, 84 with 8.
+constexpr int kShStride = 64;      // >= 55 accumulators
+constexpr int kDoneStride = 32;    // unsigned: 128 bytes
+constexpr int kMaxShParts = 8;
 
 // Counts of an entry from its 2-byte packed form, or from the full array
 // when they do not fit (o >= 255; clicked occurrences never exceed o).
@@ -115,12 +141,6 @@ constexpr uint32_t kCountsEscape = 0xFFFFu;
 __device__ __forceinline__ int2 unpack_counts(uint32_t pk, const int2* counts, int p) {
     return pk != kCountsEscape ? make_int2((int)(pk & 0xFFu), (int)(pk >> 8)) : counts[p];
 }
-// The same with the full counts `full` already loaded (the persistent
-// kernel's flush loads them for every entry slot, without a branch).
-__device__ __forceinline__ int2 unpack_counts(uint32_t pk, int2 full) {
-    return pk != kCountsEscape ? make_int2((int)(pk & 0xFFu), (int)(pk >> 8)) : full;
-}
-
 // Parameter-independent part of the M-step of per-qd table t for an entry
 // with `o` occurrences of which `c` were clicked: (prior + constant expected
 // counts, denominator).  Prior (1, 2) (utils/definitions.h:42-43); every
@@ -189,18 +209,23 @@ struct AccWindow {
     __device__ __forceinline__ int slot(int t, int q) const { return t * wstride + q; }   // q = (p << rsh) + copy
     __device__ __forceinline__ unsigned long long sum(int t, int p) const {
         if (rsh == 0) return acc[slot(t, p)];
-        unsigned long long v = 0;
-        for (int k = 0; k < (1 << rsh); k++) v += acc[slot(t, (p << rsh) + k)];
+        const unsigned long long* a = &acc[slot(t, p << rsh)];
+        if (rsh == 1) return a[0] + a[1];
+        // Four at a time: a loop of single reads waits for LDS at every copy.
+        unsigned long long v = a[0] + a[1] + a[2] + a[3];
+        for (int k = 4; k < (1 << rsh); k += 4) v += a[k] + a[k + 1] + a[k + 2] + a[k + 3];
         return v;
     }
 };
 
 // Copies per entry of a window of W entries in wstride slots: a power of
-// two, at most 64.
+// two, at most 8 (64 copies spare a few bank conflicts but are read one after
+// another in the flush: 3M uneven DBN sessions in 1,946 items 39.3 us per
+// iteration with 64, 36.1 with 8; 8M ten-rank sessions 82.4 and 82.2).
 __device__ __forceinline__ int acc_copies_log2(int W, int wstride) {
     if (W <= 0) return 0;
     const int q = wstride / W;
-    return q <= 1 ? 0 : min(6, 31 - __builtin_clz((unsigned)q));
+    return q <= 1 ? 0 : min(3, 31 - __builtin_clz((unsigned)q));
 }
 
 // --------------------------------------------------------------------------
@@ -645,6 +670,16 @@ template <> struct Shape<kUBM> { static constexpr int T = 1, K = 55, KACC = 55; 
 template <> struct Shape<kDBN> { static constexpr int T = 2, K = 1, KACC = 2; };
 template <> struct Shape<kCCM> { static constexpr int T = 1, K = 3, KACC = 6; };
 
+// Dynamic LDS of a window launch of `width` entries: accumulators and staged
+// values (the float-atomic mode's are 8 bytes an entry), then the UBM's
+// examination slots.
+inline size_t window_lds_bytes(int type, int reduce_mode, int width) {
+    const size_t T = type == kDBN ? 2 : 1;
+    if (reduce_mode != 0) return (size_t)width * T * 8;
+    const size_t b = (size_t)width * T * 12;
+    return type == kUBM ? (b + 7) / 8 * 8 + kUbmSlotBytes : b;
+}
+
 // Buffer descriptors of the session stream: 32-bit offsets (no 64-bit
 // address arithmetic per load) and hardware bounds checks (a prefetch past
 // the last session reads zeros).
@@ -743,6 +778,23 @@ __device__ __forceinline__ void decode_packed(PackedSession v, uint32_t& m, int&
 __device__ __forceinline__ long long wave_sum(long long v) {
 #pragma unroll
     for (int off = 32; off >= 1; off >>= 1) v += __shfl_xor(v, off, 64);
+    return v;
+}
+
+// Sum over the wavefront by DPP row shifts and broadcasts; valid in lane 63.
+template <int CTRL, int ROWS>
+__device__ __forceinline__ long long dpp_add(long long v) {
+    const int lo = __builtin_amdgcn_update_dpp(0, (int)(uint32_t)v, CTRL, ROWS, 0xf, true);
+    const int hi = __builtin_amdgcn_update_dpp(0, (int)(uint32_t)((unsigned long long)v >> 32), CTRL, ROWS, 0xf, true);
+    return v + (long long)(((unsigned long long)(uint32_t)hi << 32) | (uint32_t)lo);
+}
+__device__ __forceinline__ long long wave_sum_last(long long v) {
+    v = dpp_add<0x111, 0xf>(v);   // row_shr:1
+    v = dpp_add<0x112, 0xf>(v);   // row_shr:2
+    v = dpp_add<0x114, 0xf>(v);   // row_shr:4
+    v = dpp_add<0x118, 0xf>(v);   // row_shr:8
+    v = dpp_add<0x142, 0xa>(v);   // row_bcast:15 into rows 1 and 3
+    v = dpp_add<0x143, 0xc>(v);   // row_bcast:31 into rows 2 and 3
     return v;
 }
 

@@ -24,6 +24,34 @@ namespace {
 // a staged 4-byte value each: 24 KB of LDS for the DBN) unless the model's
 // MC_OPT_ITEM_WINDOW says otherwise.
 int default_window(int T) { (void)T; return 1024; }
+
+// Sessions per work item and lanes per workgroup, where the caller has not
+// set them.
+void choose_shape(mc_model* m, int64_t n, bool uneven) {
+    if (m->reduce_mode != MC_REDUCE_SEGMENTED) {
+        if (!m->block_set) m->block = 256;
+        if (!m->item_sessions_set) m->item_sessions = 8192;
+        return;
+    }
+    // PBM and CCM windows (15 KB of LDS) let eight 256-lane workgroups onto a
+    // CU; the DBN's two tables and the UBM's examination slots (30 KB) let
+    // five, so 512 lanes share a window there, and on sets too small to fill
+    // the chip, where more lanes shorten an item.  8M sessions, us per
+    // iteration with 256 / 512 lanes: PBM 69 / 81, CCM 88 / 102, DBN 87 / 83,
+    // UBM 106 / 80; 200,000 sessions: PBM 11.6 / 10.6, CCM 13.1 / 11.6.
+    // The sessions per item grow with the set so that about a thousand items
+    // (one or two per resident workgroup) hold the heavy queries: the largest
+    // item ends the launch, and each slice of a query adds its flush.  With
+    // 8192 sessions whatever the set, 32,000 PBM sessions took 31 us per
+    // iteration (256: 8), 500,000 DBN sessions 46 (1953: 15), 2M CCM sessions
+    // 72 (1953: 33).
+    const bool small_window = m->type == MC_PBM || m->type == MC_CCM;
+    if (!m->block_set) m->block = small_window && n >= 1000000 ? 256 : 512;
+    if (!m->item_sessions_set) {
+        const int64_t per = m->block >= 512 ? (uneven ? 384 : n < 1000000 ? 256 : 512) : (uneven ? 512 : 1024);
+        m->item_sessions = (int)std::min<int64_t>(16384, std::max<int64_t>(256, n / per));
+    }
+}
 }  // namespace
 
 mc_status plan_layout(mc_model* m, int64_t n, const int32_t* query, const int32_t* pidx, const uint8_t* clicks,
@@ -129,6 +157,7 @@ mc_status plan_layout(mc_model* m, int64_t n, const int32_t* query, const int32_
     //   global  slices of a group whose entries exceed W (global atomics);
     //   direct  single-session groups with distinct documents: each session
     //           owns its entries, so no reduction is needed at all.
+    choose_shape(m, n, len != nullptr);
     const int W = m->item_window > 0 ? m->item_window : default_window(T);
     const int S = m->item_sessions;
     enum { kKindWindow = 0, kKindGlobal = 1, kKindDirect = 2 };
@@ -141,7 +170,7 @@ mc_status plan_layout(mc_model* m, int64_t n, const int32_t* query, const int32_
         int32_t split = -1;     // slice of split group `split` (window slices only)
         int64_t gstart = 0;     // first session (query order) of the item's first group
     };
-    std::vector<int4> split_groups;   // per window-sliced group: first entry, end entry, slices
+    std::vector<SplitGroup> split_groups;   // per window-sliced group
     std::vector<Spec> specs;
     std::vector<int32_t> shared_idx, shared_batch;
     // Minibatches of the gradient path: contiguous runs of whole query
@@ -222,7 +251,7 @@ mc_status plan_layout(mc_model* m, int64_t n, const int32_t* query, const int32_
                     close();
                     const int64_t n_slices = (gs + S - 1) / S;
                     const int32_t split = gw <= W ? (int32_t)split_groups.size() : -1;
-                    if (gw <= W) split_groups.push_back(make_int4(g.lo, g.hi, (int)n_slices, 0));
+                    if (gw <= W) split_groups.push_back(SplitGroup{g.lo, g.hi, (int32_t)n_slices, 1, 0, 0});
                     for (int64_t k = 0; k < n_slices; k++) {
                         Spec sl;
                         const int64_t a = g.s0 + gs * k / n_slices, b = g.s0 + gs * (k + 1) / n_slices;
@@ -232,6 +261,7 @@ mc_status plan_layout(mc_model* m, int64_t n, const int32_t* query, const int32_
                         sl.width = gw <= W ? (int32_t)gw : 0;
                         sl.kind = gw <= W ? kKindWindow : kKindGlobal;
                         sl.split = split;
+                        if (split >= 0) sl.flags = (int32_t)(k << kItemSliceShift);
                         sl.gstart = g.s0;
                         specs.push_back(sl);
                     }
@@ -248,12 +278,13 @@ mc_status plan_layout(mc_model* m, int64_t n, const int32_t* query, const int32_
     if (!structured) {
         // Float atomics over uniform chunks; the merge pass finalises every entry.
         m->reduce_mode = MC_REDUCE_ATOMIC;
+        choose_shape(m, n, len != nullptr);
         specs.clear();
         shared_idx.clear();
         split_groups.clear();
-        for (int64_t a = 0; a < n; a += S) {
+        for (int64_t a = 0; a < n; a += m->item_sessions) {
             Spec c;
-            c.ranges.push_back({a, std::min<int64_t>(n, a + S)});
+            c.ranges.push_back({a, std::min<int64_t>(n, a + m->item_sessions)});
             c.count = c.ranges[0].second - a;
             c.kind = kKindGlobal;
             c.gstart = a;
@@ -396,13 +427,8 @@ mc_status plan_layout(mc_model* m, int64_t n, const int32_t* query, const int32_
     }
     m->max_item_sessions = 0;
     for (const Item& it : items) m->max_item_sessions = std::max<int64_t>(m->max_item_sessions, it.s1 - it.s0);
-    int max_width = 0;
-    for (const Item& it : items) max_width = std::max(max_width, (int)it.width);
-    m->max_width = max_width;
-    m->lds_bytes = (size_t)max_width * T * (m->reduce_mode == MC_REDUCE_SEGMENTED ? 12 : 8);
-    // The UBM's fixed-point windows are followed by its examination slots.
-    if (m->type == MC_UBM && m->reduce_mode == MC_REDUCE_SEGMENTED)
-        m->lds_bytes = (m->lds_bytes + 7) / 8 * 8 + kUbmSlotBytes;
+    m->max_width = 0;
+    for (const Item& it : items) m->max_width = std::max(m->max_width, (int)it.width);
     // ---- device layout: session records, rank-major pidx, clicks, lengths --
     // Window items come first in device order, packed ones first of all.
     // Their sessions store indices relative to the window base (the kernels

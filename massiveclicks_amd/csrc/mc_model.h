@@ -32,13 +32,13 @@ struct mc_model {
     int item_window = 1280;
     int sort_by_lcr = 1;
     int block = 256;
+    // Set by the caller; the planner chooses the others for the training set.
+    bool item_sessions_set = false, block_set = false;
     int direct = 0;
-    int persistent = 1;
     int packed = 1;           // MC_OPT_PACKED
     int skip_constant = 1;    // MC_OPT_SKIP_CONSTANT
     int fused_merge = 1;      // MC_OPT_FUSED_MERGE
-    bool fuse = false;        // the persistent kernel runs the M-step of this layout
-    int persist_grid[2] = {0, 0};   // resident workgroups of the persistent window kernel: [0] rank-major, [1] packed items
+    bool fuse = false;        // the E-step launches also run the M-step
     // shape
     int T = 1, K = 10, KACC = 10;
     int64_t N = 0, n_qd = 0;
@@ -62,9 +62,12 @@ struct mc_model {
     int max_width = 0;
     int64_t max_item_sessions = 0;
     int32_t* d_shared_idx = nullptr;
-    int4* d_split_groups = nullptr;  // per split group: first entry, end entry, slices
+    mc::SplitGroup* d_split_groups = nullptr;
+    unsigned long long* d_split_acc = nullptr;
+    int64_t n_split_acc = 0;
     unsigned* d_split_done = nullptr;
     unsigned* d_grid_done = nullptr;
+    int sh_parts = 1;                // copies of the shared-table sums (KArgs::sh_parts)
     int64_t n_shared = 0;
     float* d_val[2][2] = {{nullptr, nullptr}, {nullptr, nullptr}};   // [buf][t]
     float* d_num[2][2] = {{nullptr, nullptr}, {nullptr, nullptr}};
@@ -82,7 +85,6 @@ struct mc_model {
     unsigned long long* d_sh_acc = nullptr;
     int cur = 0;
     bool estep_pending = false;
-    size_t lds_bytes = 0;
     size_t mem_bytes = 0;
     std::vector<void*> allocations;
     // ---- gradient path (mc_grad.hip) -------------------------------------

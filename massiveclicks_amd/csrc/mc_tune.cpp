@@ -1,12 +1,11 @@
 // mc_tune.cpp -- autotuner of the EM work decomposition.
 //
 // The options that shape the E/M kernels (reduction mode, sessions per work
-// item and so sessions per lane, LDS window, persistent kernel or one
-// workgroup per item, and that workgroup's size) are picked for one model
-// type and one training set by measuring graph-replayed EM iterations of
-// each candidate on the device: first the reduction mode, then a coordinate
-// search over item size, window and launch shape, each step keeping the
-// fastest.  The starting point is a candidate, so the result is never slower
+// item and so sessions per lane, LDS window, lanes per work item) are picked
+// for one model type and one training set by measuring graph-replayed EM
+// iterations of each candidate on the device: first the reduction mode, then
+// a coordinate search over item size, window and workgroup size, each step
+// keeping the fastest.  The starting point is a candidate, so the result is never slower
 // than it (up to measurement noise).
 
 #include <cstdint>
@@ -90,17 +89,14 @@ extern "C" mc_status mc_autotune(int model_type, int device, int64_t n, const in
     if ((st = attempt(MC_OPT_REDUCE_MODE, best[MC_OPT_REDUCE_MODE] == MC_REDUCE_SEGMENTED ? MC_REDUCE_ATOMIC
                                                                                             : MC_REDUCE_SEGMENTED)) != MC_OK)
         return st;
-    for (int64_t s : {2048, 4096, 8192, 16384})
+    for (int64_t s : {512, 1024, 2048, 4096, 8192, 16384})
         if ((st = attempt(MC_OPT_ITEM_SESSIONS, s)) != MC_OK) return st;
     if (best[MC_OPT_REDUCE_MODE] == MC_REDUCE_SEGMENTED) {
         for (int64_t w : {512, 1024, 1280})
             if ((st = attempt(MC_OPT_ITEM_WINDOW, w)) != MC_OK) return st;
-        // Launch shape: the persistent kernel (256 lanes) or one workgroup per
-        // item of 256 or 512 lanes.
-        if ((st = attempt(MC_OPT_PERSISTENT, best[MC_OPT_PERSISTENT] ? 0 : 1)) != MC_OK) return st;
-        if (!best[MC_OPT_PERSISTENT])
-            for (int64_t b : {256, 512})
-                if ((st = attempt(MC_OPT_BLOCK, b)) != MC_OK) return st;
+        // Lanes per work item.
+        for (int64_t b : {256, 512})
+            if ((st = attempt(MC_OPT_BLOCK, b)) != MC_OK) return st;
         // Session format of the window items: packed records or rank-major.
         if ((st = attempt(MC_OPT_PACKED, best[MC_OPT_PACKED] ? 0 : 1)) != MC_OK) return st;
     } else {

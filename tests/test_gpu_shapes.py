@@ -1,0 +1,73 @@
+"""Work-item shapes of the EM kernels against the oracle: item counts around
+the copies of the shared sums and counters, slice counts around the copies of
+a split query group's sums, and the shapes chosen by training-set size.
+
+Bar: parameters within 1e-5 absolute of the oracle with FP64 sums after 10
+iterations (the repository's bar after 50), and bit-identical to the run with
+a separate merge kernel, whose integer sums are the same."""
+import numpy as np
+import pytest
+
+import oracle
+from massiveclicks_amd import CCM, DBN, PBM, UBM, ClickModel
+from massiveclicks_amd.model import SessionSet
+
+pytestmark = pytest.mark.gpu
+
+TOL_PARAM = 1e-5
+ITERS = 10
+IDS = {PBM: "PBM", UBM: "UBM", DBN: "DBN", CCM: "CCM"}
+
+
+def sessions(sizes, pool, seed, uneven=False):
+    """Query-grouped sessions: `sizes[q]` sessions of query q, ten of its
+    `pool` documents each; pair indices are contiguous per query."""
+    rng = np.random.default_rng(seed)
+    query = np.repeat(np.arange(len(sizes), dtype=np.int32), sizes)
+    n = len(query)
+    slot = np.argsort(rng.random((n, pool)), axis=1)[:, :10]
+    raw = query[:, None].astype(np.int64) * pool + slot
+    length = rng.integers(1, 11, n).astype(np.uint8) if uneven else None
+    shown = np.arange(10)[None, :] < (length[:, None] if uneven else np.full((n, 1), 10))
+    used, inv = np.unique(raw[shown], return_inverse=True)
+    pidx = np.full((n, 10), -1, np.int32)
+    pidx[shown] = inv
+    clicks = ((rng.random((n, 10)) < 0.25) & shown).astype(np.uint8)
+    return SessionSet(query, np.zeros((n, 10), np.int32), clicks, pidx, length), len(used)
+
+
+def check(model, train, n_qd, **opts):
+    om = oracle.OracleModel(model, train.query, np.where(train.pidx < 0, 0, train.pidx), train.clicks, n_qd,
+                            length=train.length, accum_fp64=True)
+    om.iterate(ITERS)
+    with ClickModel(model, **opts) as a, ClickModel(model, fused_merge=False, **opts) as b:
+        for cm in (a, b):
+            cm.init_parameters(train, n_qd)
+            cm.em(ITERS - 3)
+            cm.em(3, use_graph=False)
+        for t in range(a.n_tables()):
+            np.testing.assert_array_equal(a.get_parameters(t)[0], b.get_parameters(t)[0])
+            np.testing.assert_array_equal(a.get_values(t), b.get_values(t))
+            err = float(np.max(np.abs(a.get_values(t) - om.get_table(t)[2])))
+            assert err < TOL_PARAM, f"{a.layout_info()} table {t}: {err}"
+        return a.layout_info()
+
+
+@pytest.mark.parametrize("model", list(IDS), ids=IDS.get)
+@pytest.mark.parametrize("slices", [1, 2, 15, 16, 17, 33, 130, 300])
+def test_slices_of_one_query(model, slices):
+    """One query split into `slices` items of 64 sessions: one to sixteen
+    copies of the group's sums, one to eight of the shared ones."""
+    train, n_qd = sessions([64 * slices], 20, slices)
+    print(f"case slices={slices} model={model}", flush=True)
+    assert check(model, train, n_qd, item_sessions=64, block=64)["n_items"] == slices
+
+
+@pytest.mark.parametrize("model", list(IDS), ids=IDS.get)
+@pytest.mark.parametrize("sizes,uneven", [([1], False), ([3, 1, 500], True), ([40] * 31, False), ([40] * 300, True),
+                                          ([5000] + [7] * 900, False), ([30000, 200] + [2] * 3000, True)],
+                         ids=["one", "three", "31", "300", "skewed", "skewed-uneven"])
+def test_shapes_chosen_by_size(model, sizes, uneven):
+    train, n_qd = sessions(sizes, 24, len(sizes), uneven)
+    print(f"case sizes={len(sizes)} model={model} uneven={uneven}", flush=True)
+    check(model, train, n_qd)
