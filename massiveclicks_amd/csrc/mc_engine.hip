@@ -713,8 +713,10 @@ void launch_item(mc_model* m, const KArgs& A) {
         launch_path<MODEL, kPathLdsFloat>(m, A, 0, m->n_win_items, m->max_width);
         launch_path<MODEL, kPathAtomic>(m, A, m->n_win_items, m->n_glob_items, 0);
     } else {
+        const int wide = m->n_win_items - m->n_wide_items;
         launch_path<MODEL, kPathPacked>(m, A, 0, m->n_pk_items, m->max_width);
-        launch_path<MODEL, kPathLds>(m, A, m->n_pk_items, m->n_win_items - m->n_pk_items, m->max_width);
+        launch_path<MODEL, kPathLds>(m, A, m->n_pk_items, wide - m->n_pk_items, m->max_width);
+        launch_path<MODEL, kPathLds>(m, A, wide, m->n_wide_items, m->wide_width);
         launch_path<MODEL, kPathGlobal>(m, A, m->n_win_items, m->n_glob_items, 0);
         launch_path<MODEL, kPathDirect>(m, A, m->n_win_items + m->n_glob_items, m->n_dir_items, 0);
     }
@@ -831,6 +833,7 @@ mc_status mc_model_set_option(mc_model* m, int option, int64_t value) {
         case MC_OPT_ITEM_WINDOW:
             MC_REQUIRE(value >= 0 && value <= 16384, "item window out of range [0, 16384]");
             m->item_window = (int)value;
+            m->item_window_set = true;
             break;
         case MC_OPT_SORT_BY_LCR:
             m->sort_by_lcr = value != 0;
@@ -902,7 +905,7 @@ mc_status mc_init_parameters(mc_model* m, int64_t n, const int32_t* query, const
         // workgroup's LDS.
         int max_lds = 0;
         MC_HIP(hipDeviceGetAttribute(&max_lds, hipDeviceAttributeMaxSharedMemoryPerBlock, m->device));
-        const size_t lds = window_lds_bytes(m->type, m->reduce_mode, m->max_width);
+        const size_t lds = window_lds_bytes(m->type, m->reduce_mode, std::max(m->max_width, m->wide_width));
         MC_REQUIRE(lds + 4096 <= (size_t)max_lds,
                    "item window too large for this device's LDS (" + std::to_string(m->max_width) + " entries need " +
                        std::to_string(lds) + " bytes, at most " + std::to_string(max_lds) +

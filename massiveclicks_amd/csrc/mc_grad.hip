@@ -22,6 +22,7 @@
 
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <cmath>
 #include <cstring>
 #include <string>
@@ -690,7 +691,7 @@ GArgs make_gargs(mc_model* m, int batch) {
     G.steps = m->d_steps;
     G.K = m->K;
     G.kacc = m->KACC;
-    G.max_width = m->max_width;
+    G.max_width = std::max(m->max_width, m->wide_width);
     G.batch = batch < 0 ? 0 : batch;
     G.n_batches = m->n_batches;
     G.use_prior = m->adam_prior;
@@ -704,7 +705,7 @@ GArgs make_gargs(mc_model* m, int batch) {
 }
 
 // Accumulators and staged values of the widest window.
-size_t grad_lds_bytes(const mc_model* m) { return (size_t)m->max_width * m->T * 12; }
+size_t grad_lds_bytes(const mc_model* m) { return (size_t)std::max(m->max_width, m->wide_width) * m->T * 12; }
 
 template <int MODEL, bool WIN, bool ADAM, int NT>
 void launch_items(mc_model* m, const GArgs& G, int64_t count, int64_t off, size_t lds) {

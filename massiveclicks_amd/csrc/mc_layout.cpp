@@ -52,6 +52,17 @@ void choose_shape(mc_model* m, int64_t n, bool uneven) {
         m->item_sessions = (int)std::min<int64_t>(16384, std::max<int64_t>(256, n / per));
     }
 }
+
+// Entries of the widest window: with the default item window a group of more
+// entries gets a window of its own as long as two workgroups fit a CU's LDS;
+// one 64-bit atomic to L2 per shown document otherwise bounds its items.  1M
+// UBM sessions on 1,500 queries of up to 1,500 documents: 432 us per
+// iteration with global atomics, 36 us with wide windows.
+int wide_window(const mc_model* m, int W) {
+    if (m->item_window_set || m->reduce_mode != MC_REDUCE_SEGMENTED) return W;
+    const size_t budget = 78 * 1024 - window_lds_bytes(m->type, m->reduce_mode, 0);
+    return std::max<int>(W, (int)(budget / 12 / (m->type == MC_DBN ? 2 : 1)));
+}
 }  // namespace
 
 mc_status plan_layout(mc_model* m, int64_t n, const int32_t* query, const int32_t* pidx, const uint8_t* clicks,
@@ -157,10 +168,13 @@ mc_status plan_layout(mc_model* m, int64_t n, const int32_t* query, const int32_
     //   global  slices of a group whose entries exceed W (global atomics);
     //   direct  single-session groups with distinct documents: each session
     //           owns its entries, so no reduction is needed at all.
+    //   wide    (slices of) one group whose entries exceed W but fit a larger
+    //           LDS window, launched with as much LDS as they need;
     choose_shape(m, n, len != nullptr);
     const int W = m->item_window > 0 ? m->item_window : default_window(T);
     const int S = m->item_sessions;
-    enum { kKindWindow = 0, kKindGlobal = 1, kKindDirect = 2 };
+    const int W_wide = wide_window(m, W);
+    enum { kKindWindow = 0, kKindWide = 1, kKindGlobal = 2, kKindDirect = 3 };
     struct Spec {
         std::vector<std::pair<int64_t, int64_t>> ranges;
         int64_t count = 0;
@@ -249,17 +263,33 @@ mc_status plan_layout(mc_model* m, int64_t n, const int32_t* query, const int32_
                     }
                 } else {
                     close();
-                    const int64_t n_slices = (gs + S - 1) / S;
-                    const int32_t split = gw <= W ? (int32_t)split_groups.size() : -1;
-                    if (gw <= W) split_groups.push_back(SplitGroup{g.lo, g.hi, (int32_t)n_slices, 1, 0, 0});
+                    const bool wide = gw > W && gw <= W_wide;
+                    // A wide slice is at least half as many sessions as the
+                    // entries it stages and flushes.
+                    const int64_t Sg = wide ? std::max<int64_t>(S, gw / 2) : S;
+                    const int64_t n_slices = (gs + Sg - 1) / Sg;
+                    if (wide && n_slices == 1) {
+                        Spec one;
+                        one.ranges.push_back({g.s0, g.s1});
+                        one.count = gs;
+                        one.base = g.lo;
+                        one.width = (int32_t)gw;
+                        one.flags = kItemInterior;
+                        one.kind = kKindWide;
+                        one.gstart = g.s0;
+                        specs.push_back(one);
+                        continue;
+                    }
+                    const int32_t split = gw <= W_wide ? (int32_t)split_groups.size() : -1;
+                    if (gw <= W_wide) split_groups.push_back(SplitGroup{g.lo, g.hi, (int32_t)n_slices, 1, 0, 0});
                     for (int64_t k = 0; k < n_slices; k++) {
                         Spec sl;
                         const int64_t a = g.s0 + gs * k / n_slices, b = g.s0 + gs * (k + 1) / n_slices;
                         sl.ranges.push_back({a, b});
                         sl.count = b - a;
                         sl.base = g.lo;
-                        sl.width = gw <= W ? (int32_t)gw : 0;
-                        sl.kind = gw <= W ? kKindWindow : kKindGlobal;
+                        sl.width = gw <= W_wide ? (int32_t)gw : 0;
+                        sl.kind = wide ? kKindWide : gw <= W ? kKindWindow : kKindGlobal;
                         sl.split = split;
                         if (split >= 0) sl.flags = (int32_t)(k << kItemSliceShift);
                         sl.gstart = g.s0;
@@ -314,8 +344,8 @@ mc_status plan_layout(mc_model* m, int64_t n, const int32_t* query, const int32_
             if (fits) sp.flags |= kItemPacked;
         }
     }
-    // Launch order: packed window items, other window items, global items,
-    // direct items; the largest items of each kind first (workgroups are
+    // Launch order: packed window items, other window items, wide items,
+    // global items, direct items; the largest items of each kind first (workgroups are
     // dispatched in order, so long items do not end up in the tail).
     std::stable_sort(specs.begin(), specs.end(), [](const Spec& a, const Spec& b) {
         if (a.kind != b.kind) return a.kind < b.kind;
@@ -337,7 +367,7 @@ mc_status plan_layout(mc_model* m, int64_t n, const int32_t* query, const int32_
     std::vector<Item> items;
     std::vector<int64_t> order;
     order.reserve((size_t)n);
-    m->n_win_items = m->n_pk_items = m->n_glob_items = m->n_dir_items = 0;
+    m->n_win_items = m->n_pk_items = m->n_wide_items = m->n_glob_items = m->n_dir_items = 0;
     m->n_em_sessions = 0;
     for (const Spec& sp : specs) {
         const int64_t j0 = (int64_t)order.size();
@@ -357,8 +387,9 @@ mc_status plan_layout(mc_model* m, int64_t n, const int32_t* query, const int32_
         m->n_em_sessions += e1 - j0;
         items.push_back(Item{(int32_t)j0, (int32_t)order.size(), sp.base, sp.width, sp.flags, batch_of(sp.gstart),
                              (int32_t)e1, sp.split});
-        if (sp.kind == kKindWindow && structured) {
+        if ((sp.kind == kKindWindow || sp.kind == kKindWide) && structured) {
             m->n_win_items++;
+            if (sp.kind == kKindWide) m->n_wide_items++;
             if (sp.packed) m->n_pk_items++;
         }
         else if (sp.kind == kKindDirect) m->n_dir_items++;
@@ -374,7 +405,7 @@ mc_status plan_layout(mc_model* m, int64_t n, const int32_t* query, const int32_
                        "internal: work items do not tile the sessions");
             expect = it.s1;
             if (it.width > 0) {
-                MC_REQUIRE(it.base >= 0 && (int64_t)it.base + it.width <= n_qd && it.width <= W,
+                MC_REQUIRE(it.base >= 0 && (int64_t)it.base + it.width <= n_qd && it.width <= W_wide,
                            "internal: item window out of range");
                 for (int64_t j = it.s0; j < it.s1; j++) {
                     const int64_t s = order[j];
@@ -427,8 +458,11 @@ mc_status plan_layout(mc_model* m, int64_t n, const int32_t* query, const int32_
     }
     m->max_item_sessions = 0;
     for (const Item& it : items) m->max_item_sessions = std::max<int64_t>(m->max_item_sessions, it.s1 - it.s0);
-    m->max_width = 0;
-    for (const Item& it : items) m->max_width = std::max(m->max_width, (int)it.width);
+    m->max_width = m->wide_width = 0;
+    for (size_t i = 0; i < items.size(); i++) {
+        int& w = (int)i < m->n_win_items && (int)i >= m->n_win_items - m->n_wide_items ? m->wide_width : m->max_width;
+        w = std::max(w, (int)items[i].width);
+    }
     // ---- device layout: session records, rank-major pidx, clicks, lengths --
     // Window items come first in device order, packed ones first of all.
     // Their sessions store indices relative to the window base (the kernels

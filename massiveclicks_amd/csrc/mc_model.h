@@ -33,7 +33,7 @@ struct mc_model {
     int sort_by_lcr = 1;
     int block = 256;
     // Set by the caller; the planner chooses the others for the training set.
-    bool item_sessions_set = false, block_set = false;
+    bool item_sessions_set = false, item_window_set = false, block_set = false;
     int direct = 0;
     int packed = 1;           // MC_OPT_PACKED
     int skip_constant = 1;    // MC_OPT_SKIP_CONSTANT
@@ -56,10 +56,12 @@ struct mc_model {
     mc::Item* d_items = nullptr;
     int n_items = 0;
     int n_win_items = 0;      // items [0, n_win_items) have an LDS window (the first
-    int n_pk_items = 0;       //   n_pk_items of them packed),
+    int n_pk_items = 0;       //   n_pk_items of them packed, the last
+    int n_wide_items = 0;     //   n_wide_items of them wider than the item window),
     int n_glob_items = 0;     // then items merged with global atomics,
     int n_dir_items = 0;      // then direct items (single-session groups)
-    int max_width = 0;
+    int max_width = 0;        // widest window, wide items aside
+    int wide_width = 0;       // widest wide item
     int64_t max_item_sessions = 0;
     int32_t* d_shared_idx = nullptr;
     mc::SplitGroup* d_split_groups = nullptr;

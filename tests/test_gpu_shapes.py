@@ -25,7 +25,7 @@ def sessions(sizes, pool, seed, uneven=False):
     rng = np.random.default_rng(seed)
     query = np.repeat(np.arange(len(sizes), dtype=np.int32), sizes)
     n = len(query)
-    slot = np.argsort(rng.random((n, pool)), axis=1)[:, :10]
+    slot = np.argsort(rng.random((n, pool), np.float32), axis=1)[:, :10]
     raw = query[:, None].astype(np.int64) * pool + slot
     length = rng.integers(1, 11, n).astype(np.uint8) if uneven else None
     shown = np.arange(10)[None, :] < (length[:, None] if uneven else np.full((n, 1), 10))
@@ -70,4 +70,17 @@ def test_slices_of_one_query(model, slices):
 def test_shapes_chosen_by_size(model, sizes, uneven):
     train, n_qd = sessions(sizes, 24, len(sizes), uneven)
     print(f"case sizes={len(sizes)} model={model} uneven={uneven}", flush=True)
+    check(model, train, n_qd)
+
+
+@pytest.mark.parametrize("model", list(IDS), ids=IDS.get)
+@pytest.mark.parametrize("pool,sizes,uneven", [(1300, [400, 30, 5000], False), (1300, [3000, 1, 800], True),
+                                               (3400, [2500, 60, 9000], False), (7500, [6000, 300], False)],
+                         ids=["1300", "1300-uneven", "3400", "7500"])
+def test_queries_wider_than_the_item_window(model, pool, sizes, uneven):
+    """Queries of more than 1280 entries: a window of their own, whole or
+    sliced, up to what two workgroups per CU can hold (3,328 entries for the
+    DBN, 5,482 for the UBM, 6,656 for PBM and CCM), global atomics beyond."""
+    train, n_qd = sessions(sizes, pool, pool, uneven)
+    print(f"case pool={pool} model={model} uneven={uneven} n_qd={n_qd}", flush=True)
     check(model, train, n_qd)
