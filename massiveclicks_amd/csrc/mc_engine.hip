@@ -807,6 +807,14 @@ mc_status mc_model_create(int model_type, int device, mc_model** out) {
         set_error(std::string("hipStreamCreate: ") + hipGetErrorString(e));
         return MC_ERR_HIP;
     }
+    e = hipHostMalloc((void**)&m->h_totals, 21 * sizeof(double), hipHostMallocDefault);
+    if (e != hipSuccess) {
+        (void)hipGetLastError();
+        (void)hipStreamDestroy(m->stream);
+        delete m;
+        set_error(std::string("hipHostMalloc: ") + hipGetErrorString(e));
+        return MC_ERR_HIP;
+    }
     *out = m;
     return MC_OK;
 }
@@ -1049,7 +1057,7 @@ mc_status mc_em_iterations(mc_model* m, int n_iter, int use_graph) {
     MC_REQUIRE(n_iter >= 0, "n_iter must be >= 0");
     if (n_iter == 0) return MC_OK;
     MC_HIP(hipSetDevice(m->device));
-    if (use_graph) {
+    if (use_graph && n_iter > 1) {   // a graph of one launch costs more than the launch
         hipGraphExec_t g = nullptr;
         MC_TRY(get_graph(m, n_iter, m->cur, &g));
         MC_HIP(hipGraphLaunch(g, m->stream));
@@ -1282,6 +1290,7 @@ void mc_model_destroy(mc_model* m) {
     (void)hipSetDevice(m->device);
     (void)hipStreamSynchronize(m->stream);
     release(m);
+    (void)hipHostFree(m->h_totals);
     (void)hipStreamDestroy(m->stream);
     delete m;
 }

@@ -52,7 +52,7 @@ struct EvalArgs {
     float* full;             // [n][10] or null
     float* llh;              // [n] or null
     float* prob;             // [n][10] or null: get_serp_probability
-    double* partial;         // [gridDim.x][21]: llh, ppl[10], count[10]
+    double* partial;         // [21][gridDim.x]: llh, ppl[10], count[10]; the totals themselves of a single block
 };
 
 // Value of pair p, or PARAM_DEF_NUM / PARAM_DEF_DENOM = 1/2 for a pair unseen
@@ -62,24 +62,85 @@ __device__ __forceinline__ float pv_or_default(const float* v, int p, int64_t n_
     return (uint64_t)(uint32_t)p < (uint64_t)n_qd ? v[p] : 0.5f;
 }
 
-// One session's pair indices and clicks, session-major: the ten indices as
-// five 8-byte loads (rows are 40 B, so 8-byte aligned), the click bytes as
-// five 2-byte loads.
-__device__ __forceinline__ void load_session_major(const EvalArgs& E, int64_t i, int (&p)[kL], uint32_t& c) {
-    const int2* p2 = reinterpret_cast<const int2*>(E.pidx + i * kL);
+// Session-major rows of a wavefront's 64 consecutive sessions pass through
+// LDS: the wavefront reads the 64 x 40 contiguous bytes of indices and 64 x 10
+// of clicks with each instruction's lanes side by side, and a lane then takes
+// its own row from LDS; per-session outputs go the other way.  A lane reading
+// and writing its own 40-byte rows in memory touches 20 lines per instruction
+// instead of 4.
+// Pairs as the caller's arrays hold them: 4-byte words and bytes at any
+// address their element type allows.
+typedef int Pair32 __attribute__((ext_vector_type(2), aligned(4)));
+typedef uint16_t Pair8 __attribute__((aligned(1)));
+struct WaveRows {
+    int2 p[kL / 2 * 64];         // 64 rows of ten indices or floats
+    uint16_t c[kL / 2 * 64];     // 64 rows of ten click bytes
+};
+struct RowLoads {                // a wavefront's rows in flight: pair u * 64 + lane
+    int2 p[kL / 2];
+    uint16_t c[kL / 2];
+};
+
+// Orders a wavefront's own LDS accesses (LDS is in order within a wavefront;
+// this keeps the compiler from moving them).
+__device__ __forceinline__ void wave_lds_fence() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
+// Loads the rows of sessions [i0, min(i0 + 64, n)).
+__device__ __forceinline__ RowLoads load_rows(const EvalArgs& E, int64_t i0, int lane) {
+    const Pair32* p2 = reinterpret_cast<const Pair32*>(E.pidx + i0 * kL);
+    const Pair8* c2 = reinterpret_cast<const Pair8*>(E.clicks + i0 * kL);
+    const int pairs = (int)min((int64_t)64, E.n - i0) * (kL / 2);
+    RowLoads v;
 #pragma unroll
     for (int u = 0; u < kL / 2; u++) {
-        const int2 v = p2[u];
-        p[2 * u] = v.x;
-        p[2 * u + 1] = v.y;
+        const int j = min(u * 64 + lane, pairs - 1);
+        const Pair32 q = p2[j];
+        v.p[u] = make_int2(q.x, q.y);
+        v.c[u] = c2[j];
     }
-    const uint16_t* c2 = reinterpret_cast<const uint16_t*>(E.clicks + i * kL);
+    return v;
+}
+
+// This lane's session from the loaded rows, by way of LDS.
+__device__ __forceinline__ void take_row(WaveRows& w, const RowLoads& v, int lane, int (&p)[kL], uint32_t& c) {
+    wave_lds_fence();
+#pragma unroll
+    for (int u = 0; u < kL / 2; u++) {
+        w.p[u * 64 + lane] = v.p[u];
+        w.c[u * 64 + lane] = v.c[u];
+    }
+    wave_lds_fence();
     c = 0;
 #pragma unroll
     for (int u = 0; u < kL / 2; u++) {
-        const uint16_t v = c2[u];
-        c |= (uint32_t)((v & 0xffu) == 1) << (2 * u);
-        c |= (uint32_t)((v >> 8) == 1) << (2 * u + 1);
+        const int2 q = w.p[lane * (kL / 2) + u];
+        const uint32_t b = w.c[lane * (kL / 2) + u];
+        p[2 * u] = q.x;
+        p[2 * u + 1] = q.y;
+        c |= (uint32_t)((b & 0xffu) == 1) << (2 * u);
+        c |= (uint32_t)((b >> 8) == 1) << (2 * u + 1);
+    }
+}
+
+// Writes the wavefront's rows x of sessions [i0, min(i0 + 64, n)) to out.
+__device__ __forceinline__ void put_rows(WaveRows& w, float* out, int64_t i0, int64_t n, int lane, int L,
+                                         const float (&x)[kL]) {
+    wave_lds_fence();
+#pragma unroll
+    for (int u = 0; u < kL / 2; u++)
+        w.p[lane * (kL / 2) + u] = make_int2(__float_as_int(2 * u < L ? x[2 * u] : 0.f),
+                                             __float_as_int(2 * u + 1 < L ? x[2 * u + 1] : 0.f));
+    wave_lds_fence();
+    const int pairs = (int)min((int64_t)64, n - i0) * (kL / 2);
+    Pair32* o2 = reinterpret_cast<Pair32*>(out + i0 * kL);
+#pragma unroll
+    for (int u = 0; u < kL / 2; u++) {
+        const int j = u * 64 + lane;
+        if (j < pairs) o2[j] = Pair32{w.p[j].x, w.p[j].y};
     }
 }
 
@@ -254,12 +315,16 @@ __device__ __forceinline__ double wave_sum_d(double v) {
 // One session per lane, grid-stride: in every pass a wavefront takes 64
 // consecutive sessions.  Per-block FP64 partials of the 21 sums; the per-rank
 // session counts come from wavefront ballots (uniform values, no vector
-// registers).  OUT: per-session outputs requested (separate instantiation,
-// so that the common case keeps fewer values live).
-template <int MODEL, int LAYOUT, bool OUT>
+// registers).  OUT: what is asked for (separate instantiations, so that the
+// common case keeps fewer values live).
+enum { kOutTotals = 0, kOutSessions = 1, kOutProb = 2 };   // sums; sums and per-session outputs; SERP probabilities alone
+template <int MODEL, int LAYOUT, int OUT>
 __global__ void __launch_bounds__(256) eval_kernel(EvalArgs E) {
     __shared__ double red[21][4];
-    const int tid = threadIdx.x;
+    constexpr bool major = LAYOUT == kEvalSessionMajor;
+    __shared__ WaveRows rows[major ? 4 : 1];
+    const int tid = threadIdx.x, lane = tid & 63;
+    WaveRows& wr = rows[major ? tid >> 6 : 0];
     // Per-lane FP32 partials of the lane's sessions (a lane takes every
     // (blocks x 256)-th session, about four of 2M test sessions), FP64 from
     // the wavefront sums on.
@@ -269,23 +334,29 @@ __global__ void __launch_bounds__(256) eval_kernel(EvalArgs E) {
     int cnt[kL];
 #pragma unroll
     for (int r = 0; r < kL; r++) cnt[r] = 0;
-    // The next session's length, indices and clicks are in flight while a
-    // session is evaluated.
     const int64_t stride = (int64_t)gridDim.x * blockDim.x;
-    int64_t i = (int64_t)blockIdx.x * blockDim.x + tid;
+    // Session-major: i0 is the wavefront's first session (a scalar: the loads
+    // then take a scalar base and a 32-bit lane offset) and the wavefront
+    // stays together while any of its 64 sessions is left; lanes past the end
+    // hold copies of the last loads and contribute nothing.  The resident
+    // layouts keep the lane's own session in i0 (the UBM's packed kernel
+    // needs its 80 VGPRs: 42 us on 1.9M sessions, 51 with the scalar form).
+    int64_t i0 = (int64_t)blockIdx.x * blockDim.x + (major ? 64 * __builtin_amdgcn_readfirstlane(tid >> 6) : tid);
     // Packed records stay raw (4 registers) until their session is reached.
     int Ln = kL;
     int pn[kL];
     uint32_t cn = 0;
     uint4 rn = make_uint4(0u, 0u, 0u, 0u);
-    auto load = [&](int64_t j) {
+    RowLoads vn;
+    auto load = [&](int64_t j0) {
         if (LAYOUT == kEvalPacked) {
-            rn = E.packed[j];
+            rn = E.packed[j0];
             return;
         }
-        Ln = E.len ? min(max((int)E.len[j], 1), kL) : kL;
-        if (LAYOUT == kEvalRankMajor) load_rank_major(E, j, pn, cn);
-        else load_session_major(E, j, pn, cn);
+        const int u = major ? (int)min((int64_t)lane, E.n - 1 - j0) : 0;
+        Ln = E.len ? min(max((int)(E.len + j0)[u], 1), kL) : kL;
+        if (LAYOUT == kEvalRankMajor) load_rank_major(E, j0, pn, cn);
+        else vn = load_rows(E, j0, lane);
     };
     auto take = [&](int& L, uint32_t& c, float (&a)[kL], float (&sv)[kL]) {
         int p[kL];
@@ -293,39 +364,53 @@ __global__ void __launch_bounds__(256) eval_kernel(EvalArgs E) {
         c = cn;
         if (LAYOUT == kEvalPacked) {
             decode_packed_test(rn, L, p, c);
+        } else if (major) {
+            take_row(wr, vn, lane, p, c);
         } else {
 #pragma unroll
             for (int r = 0; r < kL; r++) p[r] = pn[r];
         }
         gather_values<MODEL>(E, L, p, a, sv);
     };
-    if (i < E.n) load(i);
-    for (; i < E.n; i += stride) {
+    // The resident layouts have the next session's loads in flight while one
+    // is evaluated; session-major the 15 registers they take cost more (a
+    // wavefront per SIMD: DBN 1M sessions 90 us with, 86 without).
+    if (!major && i0 < E.n) load(i0);
+    for (; i0 < E.n; i0 += stride) {
         int L;
         uint32_t c;
         float a[kL], sv[kL];
+        if (major) load(i0);
         take(L, c, a, sv);
-        if (i + stride < E.n) load(i + stride);
+        if (!major && i0 + stride < E.n) load(i0 + stride);
         float lp[kL], fp[kL], sp[kL];
-        eval_session<MODEL, OUT>(E, L, a, sv, c, lp, fp, sp);
+        eval_session<MODEL, OUT != kOutTotals>(E, L, a, sv, c, lp, fp, sp);
+        const int64_t i = major ? i0 + lane : i0;
+        const bool real = !major || i < E.n;
+        if (OUT == kOutProb) {
+            put_rows(wr, E.prob, i0, E.n, lane, L, sp);
+            continue;
+        }
         float acc = 0.f;
 #pragma unroll
         for (int r = 0; r < kL; r++)
             if (r < L) acc = acc + lp[r];
         if (!OUT) acc *= 0.693147180559945309f;   // log2 sum to natural log
         const float s = acc / L;                 // evaluation.cpp:36
-        v[0] += s;
-        const int64_t o = (OUT && LAYOUT != kEvalSessionMajor && E.perm) ? (int64_t)E.perm[i] : i;
-        if (OUT && E.llh) E.llh[o] = s;
+        if (real) v[0] += s;
+        const int64_t o = (OUT && !major && E.perm && real) ? (int64_t)E.perm[i] : i;
+        if (OUT && E.llh && real) E.llh[o] = s;
 #pragma unroll
         for (int r = 0; r < kL; r++) {
-            cnt[r] += (int)__popcll(__ballot(r < L));
-            if (r < L) v[1 + r] += log2f(fp[r]);   // evaluation.cpp:62
-            if (OUT && E.logp) E.logp[o * kL + r] = r < L ? lp[r] : 0.f;
-            if (OUT && E.full) E.full[o * kL + r] = r < L ? fp[r] : 0.f;
-            if (OUT && E.prob) E.prob[o * kL + r] = r < L ? sp[r] : 0.f;
+            cnt[r] += (int)__popcll(__ballot(r < L && real));
+            if (r < L && real) v[1 + r] += log2f(fp[r]);   // evaluation.cpp:62
+            if (OUT && !major && E.logp && real) E.logp[o * kL + r] = r < L ? lp[r] : 0.f;
+            if (OUT && !major && E.full && real) E.full[o * kL + r] = r < L ? fp[r] : 0.f;
         }
+        if (OUT && major && E.logp) put_rows(wr, E.logp, i0, E.n, lane, L, lp);
+        if (OUT && major && E.full) put_rows(wr, E.full, i0, E.n, lane, L, fp);
     }
+    if (OUT == kOutProb) return;
 #pragma unroll
     for (int k = 0; k < 11; k++) {
         double w = wave_sum_d((double)v[k]);
@@ -338,7 +423,7 @@ __global__ void __launch_bounds__(256) eval_kernel(EvalArgs E) {
     if (tid < 21) {
         double w = 0.0;
         for (int j = 0; j < (int)(blockDim.x >> 6); j++) w += red[tid][j];
-        E.partial[(int64_t)blockIdx.x * 21 + tid] = w;
+        E.partial[(int64_t)tid * gridDim.x + blockIdx.x] = w;
     }
 }
 
@@ -348,7 +433,7 @@ __global__ void __launch_bounds__(256) eval_reduce_kernel(const double* partial,
     __shared__ double red[256];
     const int k = blockIdx.x, tid = threadIdx.x;
     double w = 0.0;
-    for (int b = tid; b < n_blocks; b += 256) w += partial[(int64_t)b * 21 + k];
+    for (int b = tid; b < n_blocks; b += 256) w += partial[(int64_t)k * n_blocks + b];
     red[tid] = w;
     __syncthreads();
     for (int off = 128; off > 0; off >>= 1) {
@@ -367,8 +452,11 @@ constexpr int64_t kEvalMaxBlocks = 2048;
 // (46.1 us against 49.1 us with 2048 on the 1.94M-session set), the others
 // at or near 2048 (DBN 45.4 us; 45.9 with 1792, 46.7 with 1536, 48.0 with
 // 1024; CCM 41.3 us, 42.7 with 1536; PBM 30.6 us, 30.1 with 1792).
-int64_t eval_blocks(int64_t n, int model_type) {
-    const int64_t cap = model_type == MC_UBM ? 1536 : kEvalMaxBlocks;
+// Session-major (resident = false): 1024, one round of four workgroups per CU
+// at 99-125 VGPRs (1M sessions, us per call with 1024 / 2048: PBM 74 / 80,
+// UBM 81 / 85, CCM 70 / 76, DBN 86 / 86).
+int64_t eval_blocks(int64_t n, int model_type, bool resident) {
+    const int64_t cap = !resident ? 1024 : model_type == MC_UBM ? 1536 : kEvalMaxBlocks;
     return std::max<int64_t>(1, std::min<int64_t>((n + 255) / 256, cap));
 }
 
@@ -406,7 +494,7 @@ double* eval_scratch(int device) {
     return device >= 0 && device < kMaxDevices ? g_scratch_ptr[device] : nullptr;
 }
 
-template <int LAYOUT, bool OUT>
+template <int LAYOUT, int OUT>
 void launch_eval_out(int type, const EvalArgs& E, int64_t nb, hipStream_t s) {
     switch (type) {
         case MC_PBM: hipLaunchKernelGGL((eval_kernel<kPBM, LAYOUT, OUT>), dim3((unsigned)nb), dim3(256), 0, s, E); break;
@@ -416,11 +504,18 @@ void launch_eval_out(int type, const EvalArgs& E, int64_t nb, hipStream_t s) {
     }
 }
 
+// The evaluation and, in launch_totals, the 21 totals: a single block's
+// partials are the totals already.
 template <int LAYOUT>
-void launch_eval(int type, const EvalArgs& E, int64_t nb, hipStream_t s) {
-    if (E.logp || E.full || E.llh || E.prob) launch_eval_out<LAYOUT, true>(type, E, nb, s);
-    else launch_eval_out<LAYOUT, false>(type, E, nb, s);
+void launch_eval(int type, EvalArgs E, int64_t nb, double* out, hipStream_t s) {
+    if (nb == 1) E.partial = out;
+    if (E.logp || E.full || E.llh) launch_eval_out<LAYOUT, kOutSessions>(type, E, nb, s);
+    else launch_eval_out<LAYOUT, kOutTotals>(type, E, nb, s);
 }
+void launch_totals(const double* partial, int64_t nb, double* out, hipStream_t s) {
+    if (nb > 1) hipLaunchKernelGGL(eval_reduce_kernel, dim3(21), dim3(256), 0, s, partial, (int)nb, out);
+}
+
 
 EvalArgs model_eval_args(const mc_model* m) {
     EvalArgs E;
@@ -447,7 +542,7 @@ mc_status check_sessions(const mc_model* m, int64_t n, const int32_t* pidx, cons
     return MC_OK;
 }
 
-void unpack_totals(const double (&out)[21], double* llh_sum, double* ppl_log2_sum, int64_t* rank_count) {
+void unpack_totals(const double* out, double* llh_sum, double* ppl_log2_sum, int64_t* rank_count) {
     if (llh_sum) *llh_sum = out[0];
     for (int r = 0; r < kMaxSerp; r++) {
         if (ppl_log2_sum) ppl_log2_sum[r] = out[1 + r];
@@ -456,11 +551,11 @@ void unpack_totals(const double (&out)[21], double* llh_sum, double* ppl_log2_su
 }
 
 // Session-major evaluation of caller arrays in host memory, with temporary
-// device buffers for this call.
+// device buffers for this call; with `prob` the SERP probabilities alone.
 mc_status evaluate_host_arrays(mc_model* m, int64_t n, const int32_t* pidx, const uint8_t* clicks, const uint8_t* len,
-                               float* logp, float* full, float* llh, float* prob, double (&out)[21]) {
+                               float* logp, float* full, float* llh, float* prob) {
     MC_HIP(hipSetDevice(m->device));
-    const int64_t nb = eval_blocks(n, m->type);
+    const int64_t nb = eval_blocks(n, m->type, false);
     std::vector<void*> tmp;
     auto talloc = [&](size_t bytes) -> void* {
         void* p = nullptr;
@@ -476,10 +571,9 @@ mc_status evaluate_host_arrays(mc_model* m, int64_t n, const int32_t* pidx, cons
     float* d_fp = full ? (float*)talloc((size_t)n * kMaxSerp * 4) : nullptr;
     float* d_llh = llh ? (float*)talloc((size_t)n * 4) : nullptr;
     float* d_pr = prob ? (float*)talloc((size_t)n * kMaxSerp * 4) : nullptr;
-    double* d_part = (double*)talloc((size_t)nb * 21 * 8);
-    double* d_out = (double*)talloc(21 * 8);
+    double* d_part = prob || nb == 1 ? nullptr : (double*)talloc((size_t)nb * 21 * 8);
     if (!d_p || !d_c || (len && !d_l) || (logp && !d_lp) || (full && !d_fp) || (llh && !d_llh) || (prob && !d_pr) ||
-        !d_part || !d_out) {
+        (!prob && nb > 1 && !d_part)) {
         cleanup();
         set_error("device allocation failed in the evaluation");
         return MC_ERR_OOM;
@@ -499,11 +593,14 @@ mc_status evaluate_host_arrays(mc_model* m, int64_t n, const int32_t* pidx, cons
     E.llh = d_llh;
     E.prob = d_pr;
     E.partial = d_part;
-    launch_eval<kEvalSessionMajor>(m->type, E, nb, m->stream);
-    chk(hipGetLastError());
-    hipLaunchKernelGGL(eval_reduce_kernel, dim3(21), dim3(256), 0, m->stream, d_part, (int)nb, d_out);
-    chk(hipGetLastError());
-    chk(hipMemcpyAsync(out, d_out, 21 * 8, hipMemcpyDeviceToHost, m->stream));
+    if (prob) {
+        launch_eval_out<kEvalSessionMajor, kOutProb>(m->type, E, nb, m->stream);
+        chk(hipGetLastError());
+    } else {
+        launch_eval<kEvalSessionMajor>(m->type, E, nb, m->h_totals, m->stream);
+        launch_totals(d_part, nb, m->h_totals, m->stream);
+        chk(hipGetLastError());
+    }
     if (logp) chk(hipMemcpyAsync(logp, d_lp, (size_t)n * kMaxSerp * 4, hipMemcpyDeviceToHost, m->stream));
     if (full) chk(hipMemcpyAsync(full, d_fp, (size_t)n * kMaxSerp * 4, hipMemcpyDeviceToHost, m->stream));
     if (llh) chk(hipMemcpyAsync(llh, d_llh, (size_t)n * 4, hipMemcpyDeviceToHost, m->stream));
@@ -529,9 +626,8 @@ mc_status mc_evaluate(mc_model* m, int64_t n, const int32_t* pidx, const uint8_t
     MC_REQUIRE(m && m->initialized, "model not initialised");
     MC_REQUIRE(n >= 1 && pidx && clicks, "invalid argument");
     MC_TRY(check_sessions(m, n, pidx, clicks, len));
-    double out[21];
-    MC_TRY(evaluate_host_arrays(m, n, pidx, clicks, len, logp, full, llh, nullptr, out));
-    unpack_totals(out, llh_sum, ppl_log2_sum, rank_count);
+    MC_TRY(evaluate_host_arrays(m, n, pidx, clicks, len, logp, full, llh, nullptr));
+    unpack_totals(m->h_totals, llh_sum, ppl_log2_sum, rank_count);
     return MC_OK;
 }
 
@@ -540,8 +636,7 @@ mc_status mc_serp_probability(mc_model* m, int64_t n, const int32_t* pidx, const
     MC_REQUIRE(m && m->initialized, "model not initialised");
     MC_REQUIRE(n >= 1 && pidx && clicks && prob, "invalid argument");
     MC_TRY(check_sessions(m, n, pidx, clicks, len));
-    double out[21];
-    return evaluate_host_arrays(m, n, pidx, clicks, len, nullptr, nullptr, nullptr, prob, out);
+    return evaluate_host_arrays(m, n, pidx, clicks, len, nullptr, nullptr, nullptr, prob);
 }
 
 mc_status mc_evaluate_device(mc_model* m, int64_t n, const int32_t* pidx, const uint8_t* clicks, const uint8_t* len,
@@ -550,7 +645,7 @@ mc_status mc_evaluate_device(mc_model* m, int64_t n, const int32_t* pidx, const 
     MC_REQUIRE(pidx && clicks && totals, "null argument");
     MC_REQUIRE(n >= 1 && n <= kEvalDeviceMaxSessions,
                "n out of range [1, " + std::to_string(kEvalDeviceMaxSessions) + "] for mc_evaluate_device");
-    const int64_t nb = eval_blocks(n, m->type);
+    const int64_t nb = eval_blocks(n, m->type, false);
     MC_REQUIRE((size_t)nb * 21 <= kScratchDoubles, "internal: evaluation partials exceed the scratch array");
     double* part = eval_scratch(m->device);
     MC_REQUIRE(part, "internal: evaluation scratch not set up on this device");
@@ -564,9 +659,8 @@ mc_status mc_evaluate_device(mc_model* m, int64_t n, const int32_t* pidx, const 
     E.full = full;
     E.llh = llh;
     E.partial = part;
-    launch_eval<kEvalSessionMajor>(m->type, E, nb, m->stream);
-    MC_HIP(hipGetLastError());
-    hipLaunchKernelGGL(eval_reduce_kernel, dim3(21), dim3(256), 0, m->stream, (const double*)part, (int)nb, totals);
+    launch_eval<kEvalSessionMajor>(m->type, E, nb, totals, m->stream);
+    launch_totals(part, nb, totals, m->stream);
     MC_HIP(hipGetLastError());
     return MC_OK;
 }
@@ -653,7 +747,7 @@ mc_status mc_set_test_set(mc_model* m, int64_t n, const int32_t* pidx, const uin
     m->d_test_part = nullptr;
     m->n_test = 0;
     const size_t before = m->mem_bytes;
-    const int64_t nb = eval_blocks(n, m->type);
+    const int64_t nb = eval_blocks(n, m->type, true);
     if (packable) {
         MC_TRY(dalloc(m, &m->d_test_packed, h_pk.size() * 4));
     } else {
@@ -662,7 +756,7 @@ mc_status mc_set_test_set(mc_model* m, int64_t n, const int32_t* pidx, const uin
         if (len) MC_TRY(dalloc(m, &m->d_test_len, h_l.size()));
     }
     MC_TRY(dalloc(m, &m->d_test_perm, perm.size() * 4));
-    MC_TRY(dalloc(m, &m->d_test_part, ((size_t)nb * 21 + 21) * 8));
+    MC_TRY(dalloc(m, &m->d_test_part, (size_t)nb * 21 * 8));
     m->test_bytes = m->mem_bytes - before;
     if (packable) {
         MC_HIP(hipMemcpyAsync(m->d_test_packed, h_pk.data(), h_pk.size() * 4, hipMemcpyHostToDevice, m->stream));
@@ -683,7 +777,7 @@ mc_status mc_evaluate_test_set(mc_model* m, float* logp, float* full, float* llh
     MC_REQUIRE(m->n_test > 0, "no test set: call mc_set_test_set first");
     MC_HIP(hipSetDevice(m->device));
     const int64_t n = m->n_test;
-    const int64_t nb = eval_blocks(n, m->type);
+    const int64_t nb = eval_blocks(n, m->type, true);
     std::vector<void*> tmp;
     auto cleanup = [&]() { for (void* p : tmp) (void)hipFree(p); };
     auto talloc = [&](size_t bytes) -> float* {
@@ -711,7 +805,6 @@ mc_status mc_evaluate_test_set(mc_model* m, float* logp, float* full, float* llh
     E.full = d_fp;
     E.llh = d_llh;
     E.partial = m->d_test_part;
-    double* d_out = m->d_test_part + nb * 21;
     hipEvent_t ev[2] = {nullptr, nullptr};
     hipError_t e = hipSuccess;
     auto chk = [&](hipError_t x) { if (e == hipSuccess && x != hipSuccess) e = x; };
@@ -720,15 +813,12 @@ mc_status mc_evaluate_test_set(mc_model* m, float* logp, float* full, float* llh
         chk(hipEventCreate(&ev[1]));
         chk(hipEventRecord(ev[0], m->stream));
     }
-    if (m->d_test_packed) launch_eval<kEvalPacked>(m->type, E, nb, m->stream);
-    else launch_eval<kEvalRankMajor>(m->type, E, nb, m->stream);
+    if (m->d_test_packed) launch_eval<kEvalPacked>(m->type, E, nb, m->h_totals, m->stream);
+    else launch_eval<kEvalRankMajor>(m->type, E, nb, m->h_totals, m->stream);
     chk(hipGetLastError());
     if (kernel_ms) chk(hipEventRecord(ev[1], m->stream));
-    hipLaunchKernelGGL(eval_reduce_kernel, dim3(21), dim3(256), 0, m->stream, (const double*)m->d_test_part, (int)nb,
-                       d_out);
+    launch_totals(m->d_test_part, nb, m->h_totals, m->stream);
     chk(hipGetLastError());
-    double out[21];
-    chk(hipMemcpyAsync(out, d_out, 21 * 8, hipMemcpyDeviceToHost, m->stream));
     if (logp) chk(hipMemcpyAsync(logp, d_lp, (size_t)n * kMaxSerp * 4, hipMemcpyDeviceToHost, m->stream));
     if (full) chk(hipMemcpyAsync(full, d_fp, (size_t)n * kMaxSerp * 4, hipMemcpyDeviceToHost, m->stream));
     if (llh) chk(hipMemcpyAsync(llh, d_llh, (size_t)n * 4, hipMemcpyDeviceToHost, m->stream));
@@ -745,7 +835,7 @@ mc_status mc_evaluate_test_set(mc_model* m, float* logp, float* full, float* llh
         set_error(std::string("mc_evaluate_test_set: ") + hipGetErrorString(e));
         return MC_ERR_HIP;
     }
-    unpack_totals(out, llh_sum, ppl_log2_sum, rank_count);
+    unpack_totals(m->h_totals, llh_sum, ppl_log2_sum, rank_count);
     return MC_OK;
 }
 

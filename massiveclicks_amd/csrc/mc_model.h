@@ -125,6 +125,9 @@ struct mc_model {
     uint8_t* d_test_len = nullptr;             // [n_test] or null (10 ranks)
     int32_t* d_test_perm = nullptr;            // [n_test] caller's index of each stored session
     double* d_test_part = nullptr;             // evaluation partials and totals
+    // An evaluation's 21 totals in pinned host memory, which the kernels
+    // write: the host reads them after the synchronisation it needs anyway.
+    double* h_totals = nullptr;
     int64_t n_test = 0;
     size_t test_bytes = 0;
     // graph cache, one slot per starting buffer parity
