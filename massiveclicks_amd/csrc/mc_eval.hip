@@ -429,7 +429,9 @@ __global__ void __launch_bounds__(256) eval_kernel(EvalArgs E) {
 
 // Sums block partials: one block per output, each thread a fixed strided
 // subset, then a fixed tree; the result does not depend on scheduling.
-__global__ void __launch_bounds__(256) eval_reduce_kernel(const double* partial, int n_blocks, double* out) {
+// `running` (nullable): totals of earlier chunks, added to them.
+__global__ void __launch_bounds__(256) eval_reduce_kernel(const double* partial, int n_blocks, const double* running,
+                                                          double* out) {
     __shared__ double red[256];
     const int k = blockIdx.x, tid = threadIdx.x;
     double w = 0.0;
@@ -440,7 +442,7 @@ __global__ void __launch_bounds__(256) eval_reduce_kernel(const double* partial,
         if (tid < off) red[tid] += red[tid + off];
         __syncthreads();
     }
-    if (tid == 0) out[k] = red[0];
+    if (tid == 0) out[k] = (running ? running[k] : 0.0) + red[0];
 }
 
 // Evaluation blocks per launch: at most this many (grid-stride beyond; each
@@ -504,16 +506,16 @@ void launch_eval_out(int type, const EvalArgs& E, int64_t nb, hipStream_t s) {
     }
 }
 
-// The evaluation and, in launch_totals, the 21 totals: a single block's
-// partials are the totals already.
+// The evaluation and, in launch_totals, the 21 totals: with `out` a single
+// block's partials are the totals already.
 template <int LAYOUT>
 void launch_eval(int type, EvalArgs E, int64_t nb, double* out, hipStream_t s) {
-    if (nb == 1) E.partial = out;
+    if (nb == 1 && out) E.partial = out;
     if (E.logp || E.full || E.llh) launch_eval_out<LAYOUT, kOutSessions>(type, E, nb, s);
     else launch_eval_out<LAYOUT, kOutTotals>(type, E, nb, s);
 }
-void launch_totals(const double* partial, int64_t nb, double* out, hipStream_t s) {
-    if (nb > 1) hipLaunchKernelGGL(eval_reduce_kernel, dim3(21), dim3(256), 0, s, partial, (int)nb, out);
+void launch_totals(const double* partial, int64_t nb, const double* running, double* out, hipStream_t s) {
+    hipLaunchKernelGGL(eval_reduce_kernel, dim3(21), dim3(256), 0, s, partial, (int)nb, running, out);
 }
 
 
@@ -530,6 +532,16 @@ EvalArgs model_eval_args(const mc_model* m) {
 // Checks the caller's session arrays (session-major, host memory).
 mc_status check_sessions(const mc_model* m, int64_t n, const int32_t* pidx, const uint8_t* clicks,
                          const uint8_t* len) {
+    // One branch-free pass over everything; only what fails it (or holds
+    // anything in ranks past a session's length) is looked at one by one.
+    int32_t bad = 0;
+    const int32_t top = (int32_t)m->n_qd;
+    for (int64_t i = 0; i < n * kMaxSerp; i++) bad |= (int32_t)(pidx[i] < -1) | (int32_t)(pidx[i] >= top);
+    uint8_t bits = 0;
+    for (int64_t i = 0; i < n * kMaxSerp; i++) bits |= clicks[i];
+    if (len)
+        for (int64_t i = 0; i < n; i++) bad |= (int32_t)(len[i] < 1) | (int32_t)(len[i] > kMaxSerp);
+    if (!bad && bits <= 1) return MC_OK;
     for (int64_t i = 0; i < n; i++) {
         const int l = len ? len[i] : kMaxSerp;
         MC_REQUIRE(l >= 1 && l <= kMaxSerp, "len must be in [1, 10] (session " + std::to_string(i) + ")");
@@ -550,68 +562,81 @@ void unpack_totals(const double* out, double* llh_sum, double* ppl_log2_sum, int
     }
 }
 
-// Session-major evaluation of caller arrays in host memory, with temporary
-// device buffers for this call; with `prob` the SERP probabilities alone.
+// Session-major evaluation of caller arrays in host memory; with `prob` the
+// SERP probabilities alone.  The sessions go through the model's two pinned
+// chunks: the kernel reads a chunk's rows and writes its outputs there
+// directly (each byte crosses the link once, in whole rows), while the host
+// fills the next chunk and empties the previous one.  No device buffer is
+// allocated per session, and small calls make no copy at all.
+constexpr int64_t kEvalChunk = 16384;
 mc_status evaluate_host_arrays(mc_model* m, int64_t n, const int32_t* pidx, const uint8_t* clicks, const uint8_t* len,
                                float* logp, float* full, float* llh, float* prob) {
     MC_HIP(hipSetDevice(m->device));
-    const int64_t nb = eval_blocks(n, m->type, false);
-    std::vector<void*> tmp;
-    auto talloc = [&](size_t bytes) -> void* {
-        void* p = nullptr;
-        if (hipMalloc(&p, bytes ? bytes : 16) != hipSuccess) { (void)hipGetLastError(); return nullptr; }
-        tmp.push_back(p);
+    const int64_t chunk = std::min(n, kEvalChunk), n_chunks = (n + chunk - 1) / chunk;
+    const size_t row = (size_t)kMaxSerp * 4;
+    // Places in a pinned chunk, every one 16-byte aligned.
+    auto place = [&, at = (size_t)0](size_t bytes, bool wanted) mutable {
+        const size_t p = at;
+        if (wanted) at += (bytes + 15) / 16 * 16;
         return p;
     };
-    auto cleanup = [&]() { for (void* p : tmp) (void)hipFree(p); };
-    int32_t* d_p = (int32_t*)talloc((size_t)n * kMaxSerp * 4);
-    uint8_t* d_c = (uint8_t*)talloc((size_t)n * kMaxSerp);
-    uint8_t* d_l = len ? (uint8_t*)talloc((size_t)n) : nullptr;
-    float* d_lp = logp ? (float*)talloc((size_t)n * kMaxSerp * 4) : nullptr;
-    float* d_fp = full ? (float*)talloc((size_t)n * kMaxSerp * 4) : nullptr;
-    float* d_llh = llh ? (float*)talloc((size_t)n * 4) : nullptr;
-    float* d_pr = prob ? (float*)talloc((size_t)n * kMaxSerp * 4) : nullptr;
-    double* d_part = prob || nb == 1 ? nullptr : (double*)talloc((size_t)nb * 21 * 8);
-    if (!d_p || !d_c || (len && !d_l) || (logp && !d_lp) || (full && !d_fp) || (llh && !d_llh) || (prob && !d_pr) ||
-        (!prob && nb > 1 && !d_part)) {
-        cleanup();
-        set_error("device allocation failed in the evaluation");
-        return MC_ERR_OOM;
+    const size_t a_p = place(row * chunk, true), a_c = place((size_t)kMaxSerp * chunk, true);
+    const size_t a_l = place((size_t)chunk, len), a_lp = place(row * chunk, logp), a_fp = place(row * chunk, full);
+    const size_t a_llh = place((size_t)chunk * 4, llh), a_pr = place(row * chunk, prob);
+    MC_TRY(stage_reserve(m, place(0, true)));
+    constexpr int64_t kMaxNb = kEvalChunk / 256;
+    if (!m->d_eval_part) MC_TRY(dalloc(m, &m->d_eval_part, (size_t)(kMaxNb + 1) * 21 * 8));
+    double* running = m->d_eval_part + kMaxNb * 21;
+    auto copy_out = [&](int64_t k) -> mc_status {
+        const char* b = m->stage[k & 1];
+        const size_t at = (size_t)(k * chunk), c = (size_t)std::min(chunk, n - k * chunk);
+        MC_HIP(hipEventSynchronize(m->stage_ev[k & 1]));
+        if (logp) std::memcpy(logp + at * kMaxSerp, b + a_lp, row * c);
+        if (full) std::memcpy(full + at * kMaxSerp, b + a_fp, row * c);
+        if (llh) std::memcpy(llh + at, b + a_llh, c * 4);
+        if (prob) std::memcpy(prob + at * kMaxSerp, b + a_pr, row * c);
+        return MC_OK;
+    };
+    auto enqueue = [&](int64_t k) -> mc_status {
+        char* b = m->stage[k & 1];
+        const size_t at = (size_t)(k * chunk), c = (size_t)std::min(chunk, n - k * chunk);
+        std::memcpy(b + a_p, pidx + at * kMaxSerp, row * c);
+        std::memcpy(b + a_c, clicks + at * kMaxSerp, (size_t)kMaxSerp * c);
+        if (len) std::memcpy(b + a_l, len + at, c);
+        EvalArgs E = model_eval_args(m);
+        E.pidx = (const int32_t*)(b + a_p);
+        E.clicks = (const uint8_t*)(b + a_c);
+        E.len = len ? (const uint8_t*)(b + a_l) : nullptr;
+        E.n = (int64_t)c;
+        E.logp = logp ? (float*)(b + a_lp) : nullptr;
+        E.full = full ? (float*)(b + a_fp) : nullptr;
+        E.llh = llh ? (float*)(b + a_llh) : nullptr;
+        E.prob = prob ? (float*)(b + a_pr) : nullptr;
+        E.partial = m->d_eval_part;
+        const int64_t nb = eval_blocks((int64_t)c, m->type, false);
+        if (prob) {
+            launch_eval_out<kEvalSessionMajor, kOutProb>(m->type, E, nb, m->stream);
+        } else if (n_chunks == 1) {
+            launch_eval<kEvalSessionMajor>(m->type, E, nb, m->h_totals, m->stream);
+            if (nb > 1) launch_totals(m->d_eval_part, nb, nullptr, m->h_totals, m->stream);
+        } else {
+            launch_eval<kEvalSessionMajor>(m->type, E, nb, nullptr, m->stream);
+            launch_totals(m->d_eval_part, nb, k > 0 ? running : nullptr, k == n_chunks - 1 ? m->h_totals : running,
+                          m->stream);
+        }
+        MC_HIP(hipGetLastError());
+        MC_HIP(hipEventRecord(m->stage_ev[k & 1], m->stream));
+        return MC_OK;
+    };
+    mc_status st = MC_OK;
+    for (int64_t k = 0; k < n_chunks && st == MC_OK; k++) {
+        if (k >= 2) st = copy_out(k - 2);
+        if (st == MC_OK) st = enqueue(k);
     }
-    hipError_t e = hipSuccess;
-    auto chk = [&](hipError_t x) { if (e == hipSuccess && x != hipSuccess) e = x; };
-    chk(hipMemcpyAsync(d_p, pidx, (size_t)n * kMaxSerp * 4, hipMemcpyHostToDevice, m->stream));
-    chk(hipMemcpyAsync(d_c, clicks, (size_t)n * kMaxSerp, hipMemcpyHostToDevice, m->stream));
-    if (len) chk(hipMemcpyAsync(d_l, len, (size_t)n, hipMemcpyHostToDevice, m->stream));
-    EvalArgs E = model_eval_args(m);
-    E.pidx = d_p;
-    E.clicks = d_c;
-    E.len = d_l;
-    E.n = n;
-    E.logp = d_lp;
-    E.full = d_fp;
-    E.llh = d_llh;
-    E.prob = d_pr;
-    E.partial = d_part;
-    if (prob) {
-        launch_eval_out<kEvalSessionMajor, kOutProb>(m->type, E, nb, m->stream);
-        chk(hipGetLastError());
-    } else {
-        launch_eval<kEvalSessionMajor>(m->type, E, nb, m->h_totals, m->stream);
-        launch_totals(d_part, nb, m->h_totals, m->stream);
-        chk(hipGetLastError());
-    }
-    if (logp) chk(hipMemcpyAsync(logp, d_lp, (size_t)n * kMaxSerp * 4, hipMemcpyDeviceToHost, m->stream));
-    if (full) chk(hipMemcpyAsync(full, d_fp, (size_t)n * kMaxSerp * 4, hipMemcpyDeviceToHost, m->stream));
-    if (llh) chk(hipMemcpyAsync(llh, d_llh, (size_t)n * 4, hipMemcpyDeviceToHost, m->stream));
-    if (prob) chk(hipMemcpyAsync(prob, d_pr, (size_t)n * kMaxSerp * 4, hipMemcpyDeviceToHost, m->stream));
-    chk(hipStreamSynchronize(m->stream));
-    cleanup();
-    if (e != hipSuccess) {
-        set_error(std::string("evaluation: ") + hipGetErrorString(e));
-        return MC_ERR_HIP;
-    }
-    return MC_OK;
+    for (int64_t k = std::max<int64_t>(0, n_chunks - 2); k < n_chunks && st == MC_OK; k++) st = copy_out(k);
+    const hipError_t e = hipStreamSynchronize(m->stream);
+    if (st == MC_OK) MC_HIP(e);
+    return st;
 }
 
 }  // namespace mc
@@ -660,7 +685,7 @@ mc_status mc_evaluate_device(mc_model* m, int64_t n, const int32_t* pidx, const 
     E.llh = llh;
     E.partial = part;
     launch_eval<kEvalSessionMajor>(m->type, E, nb, totals, m->stream);
-    launch_totals(part, nb, totals, m->stream);
+    if (nb > 1) launch_totals(part, nb, nullptr, totals, m->stream);
     MC_HIP(hipGetLastError());
     return MC_OK;
 }
@@ -817,11 +842,12 @@ mc_status mc_evaluate_test_set(mc_model* m, float* logp, float* full, float* llh
     else launch_eval<kEvalRankMajor>(m->type, E, nb, m->h_totals, m->stream);
     chk(hipGetLastError());
     if (kernel_ms) chk(hipEventRecord(ev[1], m->stream));
-    launch_totals(m->d_test_part, nb, m->h_totals, m->stream);
+    if (nb > 1) launch_totals(m->d_test_part, nb, nullptr, m->h_totals, m->stream);
     chk(hipGetLastError());
-    if (logp) chk(hipMemcpyAsync(logp, d_lp, (size_t)n * kMaxSerp * 4, hipMemcpyDeviceToHost, m->stream));
-    if (full) chk(hipMemcpyAsync(full, d_fp, (size_t)n * kMaxSerp * 4, hipMemcpyDeviceToHost, m->stream));
-    if (llh) chk(hipMemcpyAsync(llh, d_llh, (size_t)n * 4, hipMemcpyDeviceToHost, m->stream));
+    mc_status st = MC_OK;
+    if (logp && e == hipSuccess) st = download(m, logp, d_lp, (size_t)n * kMaxSerp * 4);
+    if (full && e == hipSuccess && st == MC_OK) st = download(m, full, d_fp, (size_t)n * kMaxSerp * 4);
+    if (llh && e == hipSuccess && st == MC_OK) st = download(m, llh, d_llh, (size_t)n * 4);
     chk(hipStreamSynchronize(m->stream));
     if (kernel_ms && e == hipSuccess) {
         float ms = 0.f;
@@ -835,6 +861,7 @@ mc_status mc_evaluate_test_set(mc_model* m, float* logp, float* full, float* llh
         set_error(std::string("mc_evaluate_test_set: ") + hipGetErrorString(e));
         return MC_ERR_HIP;
     }
+    if (st != MC_OK) return st;
     unpack_totals(m->h_totals, llh_sum, ppl_log2_sum, rank_count);
     return MC_OK;
 }

@@ -916,19 +916,19 @@ mc_status mc_loglik_gradient(mc_model* m, int batch, double* loglik, float* cons
     for (int t = 0; t < m->T; t++) MC_TRY(fill(m, m->d_grad[t], 0.f, m->n_qd));
     MC_TRY(fill(m, (float*)m->d_ll_part, 0.f, 2 * (int64_t)m->n_items));
     MC_TRY(launch_grad(m, batch, false));
-    MC_HIP(hipStreamSynchronize(m->stream));
     if (loglik) {
         std::vector<double> part((size_t)m->n_items);
-        MC_HIP(hipMemcpy(part.data(), m->d_ll_part, part.size() * 8, hipMemcpyDeviceToHost));
+        MC_TRY(download(m, part.data(), m->d_ll_part, part.size() * 8));
         double s = 0.0;
         for (double v : part) s += v;
         *loglik = s;
     }
     if (grad) {
         for (int t = 0; t < m->T; t++)
-            if (grad[t]) MC_HIP(hipMemcpy(grad[t], m->d_grad[t], (size_t)m->n_qd * 4, hipMemcpyDeviceToHost));
-        if (grad[m->T]) MC_HIP(hipMemcpy(grad[m->T], m->d_sh_grad, (size_t)m->K * 4, hipMemcpyDeviceToHost));
+            if (grad[t]) MC_TRY(download(m, grad[t], m->d_grad[t], (size_t)m->n_qd * 4));
+        if (grad[m->T]) MC_TRY(download(m, grad[m->T], m->d_sh_grad, (size_t)m->K * 4));
     }
+    MC_HIP(hipStreamSynchronize(m->stream));
     return MC_OK;
 }
 
@@ -988,11 +988,8 @@ mc_status mc_get_logits(mc_model* m, int t, float* logits) {
     MC_REQUIRE(m && m->initialized && logits && t >= 0 && t <= m->T, "invalid argument");
     MC_REQUIRE(m->grad_ready, "call mc_grad_init first");
     MC_HIP(hipSetDevice(m->device));
-    MC_HIP(hipStreamSynchronize(m->stream));
     const bool sh = t == m->T;
-    MC_HIP(hipMemcpy(logits, sh ? m->d_sh_logit : m->d_logit[t], (size_t)(sh ? m->K : m->n_qd) * 4,
-                     hipMemcpyDeviceToHost));
-    return MC_OK;
+    return download(m, logits, sh ? m->d_sh_logit : m->d_logit[t], (size_t)(sh ? m->K : m->n_qd) * 4);
 }
 
 mc_status mc_set_logits(mc_model* m, int t, const float* logits) {

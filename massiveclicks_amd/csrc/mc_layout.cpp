@@ -106,7 +106,6 @@ mc_status plan_layout(mc_model* m, int64_t n, const int32_t* query, const int32_
         MC_REQUIRE(occ[p] < INT32_MAX, "too many occurrences of one query-document pair");
         counts[p] = make_int2((int)occ[p], (int)clk[p]);
     }
-    m->h_counts = counts;
     std::vector<double> sh_base(2 * (size_t)K, 0.0);
     std::vector<int32_t> sh_map(2 * (size_t)K, -1);
     switch (m->type) {

@@ -21,6 +21,10 @@
         }                                                                                     \
     } while (0)
 
+namespace mc {
+constexpr int kStages = 8;         // pinned chunks of a model
+constexpr int kStageThreads = 4;   // threads that copy out of them
+}
 
 struct mc_model {
     int type = 0;
@@ -75,7 +79,6 @@ struct mc_model {
     float* d_num[2][2] = {{nullptr, nullptr}, {nullptr, nullptr}};
     int2* d_counts = nullptr;
     uint16_t* d_counts16 = nullptr;  // packed counts read by the window flushes
-    std::vector<int2> h_counts;   // host copy (occurrences, clicked) per entry
     unsigned long long* d_gacc[2] = {nullptr, nullptr};
     float* d_den_user[2] = {nullptr, nullptr};
     int den_state[3] = {0, 0, 0};  // per table: 0 prior (2), 1 user-set, 2 M-step constant, 3 value only
@@ -89,6 +92,12 @@ struct mc_model {
     bool estep_pending = false;
     size_t mem_bytes = 0;
     std::vector<void*> allocations;
+    // Pinned host chunks of stage_cap bytes through which results leave the
+    // device (and the sessions of host-array evaluations enter it), one
+    // allocation made by the first call that needs them.
+    char* stage[mc::kStages] = {};
+    size_t stage_cap = 0;
+    hipEvent_t stage_ev[mc::kStages] = {};
     // ---- gradient path (mc_grad.hip) -------------------------------------
     int n_batches = 1;             // MC_OPT_BATCHES: minibatches of whole query groups
     std::vector<int64_t> batch_sessions;       // sessions per batch
@@ -129,6 +138,7 @@ struct mc_model {
     // write: the host reads them after the synchronisation it needs anyway.
     double* h_totals = nullptr;
     int64_t n_test = 0;
+    double* d_eval_part = nullptr;             // partials and running totals of host-array evaluations
     size_t test_bytes = 0;
     // graph cache, one slot per starting buffer parity
     hipGraphExec_t graph[2] = {nullptr, nullptr};
@@ -157,6 +167,11 @@ inline mc_status dalloc(mc_model* m, P** ptr, size_t bytes) {
 void release(mc_model* m);
 // Fills n floats with v on m's stream (a kernel, safe inside graph capture).
 mc_status fill(mc_model* m, float* p, float v, int64_t n);
+// Pinned chunks of at least `bytes` each.
+mc_status stage_reserve(mc_model* m, size_t bytes);
+// Copies n bytes from the device to pageable host memory, after the work
+// enqueued on m's stream, and waits.
+mc_status download(mc_model* m, void* dst, const void* src, size_t n);
 const char* table_name(int type, int t);
 // Resolves, once per device, the device address of the evaluation scratch
 // array of mc_evaluate_device (mc_eval.hip); called by mc_model_create with

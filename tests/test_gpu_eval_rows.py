@@ -1,6 +1,7 @@
 """Session-major evaluation around its wavefront and block edges: the rows
 of a wavefront pass through LDS, so partial wavefronts, a single block (whose
-partials are the totals) and arrays at odd addresses are what can go wrong.
+partials are the totals), the chunks that host arrays are cut into and arrays at
+odd addresses are what can go wrong.
 
 Bar: per-session values bit-identical to the resident set's kernels, which
 share the per-session arithmetic; totals within 1e-6 relative (FP32 partials
@@ -17,7 +18,7 @@ from test_zz_no_alloc import Hip
 pytestmark = pytest.mark.gpu
 
 NAMES = {PBM: "pbm", UBM: "ubm", DBN: "dbn", CCM: "ccm"}
-SIZES = [1, 2, 63, 64, 65, 255, 256, 257, 1000, 262_143, 262_145]
+SIZES = [1, 2, 63, 64, 65, 255, 256, 257, 1000, 16_384, 16_385, 32_769, 49_152, 262_145]
 _models = {}
 
 
