@@ -672,11 +672,14 @@ namespace {
 constexpr size_t kStageChunk = (size_t)1 << 20;
 constexpr size_t kStageSmallChunk = (size_t)256 << 10;
 constexpr size_t kStageThreadsFrom = (size_t)8 << 20;   // below, starting threads costs more than they save
+// About four chunks of a small array, so that copies overlap.
+size_t stage_chunk(size_t n) {
+    return std::min(n, std::min(kStageChunk, std::max(kStageSmallChunk, (n / 4 + 255) / 256 * 256)));
+}
 template <class Produce>
 mc_status staged_out(mc_model* m, char* dst, size_t n, Produce produce) {
     if (n == 0) return MC_OK;
-    // About four chunks of a small array, so that copies overlap.
-    const size_t chunk = std::min(n, std::min(kStageChunk, std::max(kStageSmallChunk, (n / 4 + 255) / 256 * 256)));
+    const size_t chunk = stage_chunk(n);
     MC_TRY(stage_reserve(m, chunk));
     const size_t chunks = (n + chunk - 1) / chunk;
     auto size_of = [&](size_t k) { return std::min(chunk, n - k * chunk); };
@@ -1151,6 +1154,7 @@ mc_status mc_init_parameters(mc_model* m, int64_t n, const int32_t* query, const
         MC_TRY(fill(m, m->d_sh_den[b], 2.f, K));
     }
     m->den_state[T] = 0;
+    MC_TRY(stage_reserve(m, stage_chunk((size_t)n_qd * 4)));   // for the tables' readback
     MC_HIP(hipStreamSynchronize(m->stream));
     m->cur = 0;
     m->estep_pending = false;

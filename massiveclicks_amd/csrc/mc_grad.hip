@@ -87,29 +87,53 @@ struct GArgs {
     const unsigned long long* prev_acc;
     unsigned long long* zero_acc;  // shared sums cleared by workgroup 0 (read two steps ago)
     int32_t K, kacc, max_width, batch, n_batches, use_prior;
+    int32_t end_epoch;             // the merge of an epoch's last batch
     float lr, b1, b2, eps;
     double sh_scale;               // training sessions / batch sessions
 };
 
-// Signed 32.32 fixed point (two's complement), saturating at +-2^30.
+// Signed 32.32 fixed point (two's complement), rounding down, saturating at
+// +-2^30 (a NaN becomes -2^30).  The fraction of a tiny negative x rounds to
+// 1, which the saturating conversion takes to 1 - 2^-32 (asm: out of range it
+// is undefined in C++).
 __device__ __forceinline__ long long to_fix_signed(float x) {
-    x = fminf(fmaxf(x, -1073741824.f), 1073741824.f);
+    x = __builtin_amdgcn_fmed3f(x, -1073741824.f, 1073741824.f);
     const float fl = floorf(x);
     const int hi = (int)fl;
-    const uint32_t lo = (uint32_t)((x - fl) * kFixScale);
+    uint32_t lo;
+    asm("v_cvt_u32_f32 %0, %1" : "=v"(lo) : "v"((x - fl) * kFixScale));
     return (long long)(((unsigned long long)(long long)hi << 32) | lo);
+}
+
+// To nearest, for |x| < 2^18 (else to_fix_signed): adding 1.5 x 2^20 in FP64
+// leaves x in 32.32 fixed point in the low bits of the sum, so only the
+// constant's exponent has to come off the high word.
+__device__ __forceinline__ unsigned long long to_fix_near(float x) {
+    if (__builtin_expect(!(fabsf(x) < 262144.f), 0)) return (unsigned long long)to_fix_signed(x);
+    const double d = (double)x + 1572864.0;   // 1.5 x 2^20: high word 0x41380000, low word 0
+    return (unsigned long long)__double_as_longlong(d) - 0x4138000000000000ull;
 }
 
 __device__ __forceinline__ double fix_to_double(unsigned long long v) { return (double)(long long)v * kFixInv; }
 
 template <int T>
-struct EmitLdsSigned {
-    unsigned long long* acc;
-    __device__ __forceinline__ void add(int t, int, int p, float x) {
-        atomicAdd(&acc[p * T + t], (unsigned long long)to_fix_signed(x));
+struct EmitLdsSigned {             // as EmitLds: this lane's copies of the window's entries and of the UBM's slots
+    static constexpr bool kSlotsInLds = true;
+    char* base[T];
+    int sh;
+    unsigned long long* slots;
+    __device__ __forceinline__ EmitLdsSigned(const AccWindow<T>& w, int copy, unsigned long long* lane_slots)
+        : sh(w.rsh + 3), slots(lane_slots) {
+#pragma unroll
+        for (int t = 0; t < T; t++) base[t] = (char*)&w.acc[w.slot(t, copy)];
     }
+    __device__ __forceinline__ void add(int t, int, int p, float x) {
+        atomicAdd((unsigned long long*)(base[t] + (p << sh)), (unsigned long long)to_fix_signed(x));
+    }
+    __device__ __forceinline__ void add_slot(int k, float x) { atomicAdd(&slots[k * kUbmCopies], to_fix_near(x)); }
 };
 struct EmitGlobalSigned {
+    static constexpr bool kSlotsInLds = false;
     unsigned long long* g0;
     unsigned long long* g1;
     __device__ __forceinline__ void add(int t, int, int p, float x) {
@@ -132,14 +156,14 @@ __device__ __forceinline__ float sigmoid(float x) { return 1.f / (1.f + __expf(-
 template <int MODEL, bool VARLEN, bool LL, class Src, class Emit>
 __device__ __forceinline__ void grad_pbm_ubm(const int (&pv)[kL], int L, uint32_t mm, const Src& src, Emit& em,
                                              const float* sh, float (&acc)[55], float& ll) {
-    int slot[kL];
-    if (MODEL == kUBM) ubm_slots(mm, slot);
+    int prev = kL - 1;   // previous click (UBM), kL - 1 until the first
 #pragma unroll
     for (int r = 0; r < kL; r++) {
         if (VARLEN && r >= L) continue;
         const int p = pv[r];
         const float a = src.get(0, p);
-        const float e = MODEL == kUBM ? sh[slot[r]] : sh[r];
+        const int row = r * (r + 1) / 2, slot = row + prev;
+        const float e = MODEL == kUBM ? sh[slot] : sh[r];
         const float ae = a * e;
         float ge;
         if ((mm >> r) & 1u) {
@@ -153,10 +177,17 @@ __device__ __forceinline__ void grad_pbm_ubm(const int (&pv)[kL], int L, uint32_
             ge = -w * (1.f - e);
         }
         if (MODEL == kUBM) {
-            const int row = r * (r + 1) / 2;
+            if constexpr (Emit::kSlotsInLds) {
+                // The row's "no earlier click" slot in a register, the others
+                // one LDS add (as in the E-step).
+                if (prev == kL - 1) acc[row + kL - 1] += ge;
+                else em.add_slot(slot, ge);
+            } else {
 #pragma unroll
-            for (int j = 0; j < r; j++) acc[row + j] += (slot[r] == row + j) ? ge : 0.f;
-            acc[row + kL - 1] += (slot[r] == row + kL - 1) ? ge : 0.f;
+                for (int j = 0; j < r; j++) acc[row + j] += (slot == row + j) ? ge : 0.f;
+                acc[row + kL - 1] += (slot == row + kL - 1) ? ge : 0.f;
+            }
+            prev = ((mm >> r) & 1u) ? r : prev;
         } else {
             acc[r] += ge;
         }
@@ -349,13 +380,16 @@ __global__ void __launch_bounds__(NT) grad_item_kernel(GArgs G, int64_t list_off
     __shared__ float sh[K < 64 ? 64 : K];
     __shared__ long long red[K][NW];
     __shared__ double lred[NW];
+    constexpr bool lslots = MODEL == kUBM && WIN;   // UBM examination slots in LDS after the window
 
     const int item_idx = G.lists[list_off + blockIdx.x];
     const Item it = G.items[item_idx];
     const int tid = threadIdx.x;
     const int W = WIN ? it.width : 0;
-    unsigned long long* lacc = lds;
+    const AccWindow<T> aw{lds, G.max_width, acc_copies_log2(W, G.max_width)};
+    const int WS = W << aw.rsh;
     float* lval = (float*)(lds + T * G.max_width);
+    unsigned long long* slots = lds + ((size_t)T * G.max_width * 12 + 7) / 8;
 
     KArgs ka;
     ka.packed = G.packed;
@@ -389,11 +423,31 @@ __global__ void __launch_bounds__(NT) grad_item_kernel(GArgs G, int64_t list_off
             merge_split_entry<MODEL, true>(G, G.prev_off, i, pad);
     }
     if (WIN) {
-        for (int i = tid; i < W; i += NT) {
+        // The first values in flight while the accumulators are cleared.
+        constexpr int U = 1280 / NT + 1;
+        for (int i0 = 0; i0 < W; i0 += U * NT) {
+            float v[U][T];
 #pragma unroll
-            for (int t = 0; t < T; t++) {
-                lacc[i * T + t] = 0ull;
-                lval[i * T + t] = G.val[t][it.base + i];
+            for (int u = 0; u < U; u++) {
+                if (i0 + u * NT >= W) break;
+                const int i = min(i0 + u * NT + tid, W - 1);
+#pragma unroll
+                for (int t = 0; t < T; t++) v[u][t] = G.val[t][it.base + i];
+            }
+            if (i0 == 0) {
+                for (int i = tid; i < WS; i += NT)
+#pragma unroll
+                    for (int t = 0; t < T; t++) lds[aw.slot(t, i)] = 0ull;
+                if (lslots)
+                    for (int i = tid; i < kUbmSlots * kUbmCopies; i += NT) slots[i] = 0ull;
+            }
+#pragma unroll
+            for (int u = 0; u < U; u++) {
+                const int i = i0 + u * NT + tid;
+                if (i0 + u * NT >= W) break;
+#pragma unroll
+                for (int t = 0; t < T; t++)
+                    if (i < W) lval[i * T + t] = v[u][t];
             }
         }
     }
@@ -427,7 +481,7 @@ __global__ void __launch_bounds__(NT) grad_item_kernel(GArgs G, int64_t list_off
     {
         const SrcLds<T> lsrc{lval};
         const SrcGlobal gsrc{G.val[0], G.val[1]};
-        EmitLdsSigned<T> el{lacc};
+        EmitLdsSigned<T> el{aw, tid & ((1 << aw.rsh) - 1), slots + (tid & (kUbmCopies - 1))};
         EmitGlobalSigned eg{G.gacc[0], G.gacc[1]};
         if (packed) {
             for (int s = it.s0 + tid; s < it.s1; s += NT) {
@@ -454,17 +508,40 @@ __global__ void __launch_bounds__(NT) grad_item_kernel(GArgs G, int64_t list_off
     // Shared tables and the log-likelihood: wave sums, then one atomic per
     // accumulator and item.
     const int wave = tid >> 6, lane = tid & 63;
+    if constexpr (lslots) {
+        unsigned long long* mine = slots + (tid & (kUbmCopies - 1));
 #pragma unroll
-    for (int k = 0; k < K; k++) {
-        const long long v = wave_sum(to_fix_signed(acc[k]));
-        if (lane == 0) red[k][wave] = v;
+        for (int r = 0; r < kL; r++) {
+            const int k = r * (r + 1) / 2 + kL - 1;
+            if (acc[k] != 0.f) atomicAdd(&mine[k * kUbmCopies], (unsigned long long)to_fix_signed(acc[k]));
+        }
+    } else {
+#pragma unroll
+        for (int k = 0; k < K; k++) {
+            const long long v = wave_sum_last(to_fix_signed(acc[k]));
+            if (lane == 63) red[k][wave] = v;
+        }
     }
     if (!ADAM) {
         const double lw = wave_sum_f64((double)ll);
         if (lane == 0) lred[wave] = lw;
     }
     __syncthreads();
-    for (int k = tid; k < K; k += NT) {
+    if constexpr (lslots) {   // eight lanes add up each slot's copies
+        for (int q = tid; q < 8 * ((kUbmSlots + 7) / 8 * 8); q += NT) {
+            const int k = q >> 3, c = q & 7;
+            long long v = 0;
+            if (k < kUbmSlots)
+#pragma unroll
+                for (int j = 0; j < kUbmCopies / 8; j++) v += (long long)slots[k * kUbmCopies + c + 8 * j];
+            v += __shfl_xor(v, 1, 64);
+            v += __shfl_xor(v, 2, 64);
+            v += __shfl_xor(v, 4, 64);
+            if (c == 0 && k < kUbmSlots && v != 0)
+                atomicAdd(&G.sh_acc[(blockIdx.x % kShParts) * kShAccStride + k], (unsigned long long)v);
+        }
+    }
+    for (int k = lslots ? K : tid; k < K; k += NT) {
         long long v = 0;
 #pragma unroll
         for (int w = 0; w < NW; w++) v += red[k][w];
@@ -488,7 +565,7 @@ __global__ void __launch_bounds__(NT) grad_item_kernel(GArgs G, int64_t list_off
             const int2 oc = unpack_counts(f_oc[u], G.counts, p);
 #pragma unroll
             for (int t = 0; t < T; t++) {
-                const float g = entry_gradient<MODEL>(t, fix_to_double(lacc[i * T + t]), oc, lval[i * T + t],
+                const float g = entry_gradient<MODEL>(t, fix_to_double(aw.sum(t, i)), oc, lval[i * T + t],
                                                       ADAM && G.use_prior);
                 if (ADAM) {
                     G.val[t][p] = ad.apply(f_logit[u][t], f_m[u][t], f_v[u][t], g);
@@ -527,7 +604,7 @@ __global__ void __launch_bounds__(NT) grad_item_kernel(GArgs G, int64_t list_off
                 const int2 ocu = interior ? unpack_counts(oc[u], G.counts, p) : make_int2(0, 0);
 #pragma unroll
                 for (int t = 0; t < T; t++) {
-                    const unsigned long long v = lacc[i * T + t];
+                    const unsigned long long v = aw.sum(t, i);
                     if (interior) {
                         const float g = entry_gradient<MODEL>(t, fix_to_double(v), ocu, lval[i * T + t],
                                                               ADAM && G.use_prior);
@@ -549,8 +626,9 @@ __global__ void __launch_bounds__(NT) grad_item_kernel(GArgs G, int64_t list_off
 }
 
 // Block 0: the shared tables (gradient scaled to the training set, prior,
-// Adam); other blocks: the listed split entries.  With Adam, the last block
-// to finish advances the step counts, after every block has read them.
+// Adam); other blocks: the listed split entries.  A single block does both
+// and, after a batch that ends an epoch (G.end_epoch), counts the epoch: a
+// launch fewer per epoch (4 us).
 template <int MODEL, bool ADAM>
 __global__ void __launch_bounds__(256) grad_merge_kernel(GArgs G) {
     const int tid = threadIdx.x;
@@ -560,6 +638,14 @@ __global__ void __launch_bounds__(256) grad_merge_kernel(GArgs G) {
         for (int j = tid; j < kShAccSlot; j += blockDim.x) G.sh_acc[j] = 0ull;
         if (G.zero_acc)
             for (int j = tid; j < 3 * kShAccSlot; j += blockDim.x) G.zero_acc[j] = 0ull;
+        if (gridDim.x == 1) {
+            AdamStep ad;
+            if (ADAM) ad = adam_step(G, G.steps[0] + 1);
+            for (int64_t i = tid; i < G.shared_cnt; i += blockDim.x)
+                merge_split_entry<MODEL, ADAM>(G, G.shared_off, i, ad);
+            __syncthreads();
+            if (ADAM && G.end_epoch && tid == 0) G.steps[0] += 1;
+        }
     } else {
         const int64_t i = (int64_t)(blockIdx.x - 1) * blockDim.x + tid;
         AdamStep ad;
@@ -704,8 +790,21 @@ GArgs make_gargs(mc_model* m, int batch) {
     return G;
 }
 
-// Accumulators and staged values of the widest window.
-size_t grad_lds_bytes(const mc_model* m) { return (size_t)std::max(m->max_width, m->wide_width) * m->T * 12; }
+// Accumulators and staged values of the widest window, the UBM's slots.
+size_t grad_lds_bytes(const mc_model* m) {
+    return window_lds_bytes(m->type, MC_REDUCE_SEGMENTED, std::max(m->max_width, m->wide_width));
+}
+
+// 1024 lanes per item where a launch has few items (a small minibatch: one
+// workgroup per CU then), else 512, which keep 24 to 32 wavefronts on a CU.
+// Adam epochs, us with 1024 / 512 lanes: 700,000 DBN sessions in 729 items
+// 46.5 / 35.5; 1M in three minibatches of 200 items 94 / 119; 256 lanes took
+// 20 more of 126 us on the 1,360 items of the rarest queries.  Items of more
+// than 4096 sessions stay with 1024 lanes up to four per CU (a gradient of 1M
+// sessions in 605 items of up to 8192: 53 / 63 us).
+bool wide_items(const mc_model* m, int64_t n_items) {
+    return 2 * n_items < 3 * (int64_t)m->n_cu || (n_items < 4 * (int64_t)m->n_cu && m->max_item_sessions > 4096);
+}
 
 template <int MODEL, bool WIN, bool ADAM, int NT>
 void launch_items(mc_model* m, const GArgs& G, int64_t count, int64_t off, size_t lds) {
@@ -717,6 +816,16 @@ void launch_items(mc_model* m, const GArgs& G, int64_t count, int64_t off, size_
                            m->stream, G, off);
 }
 
+// The merge in one block while that takes one pass over its split entries,
+// and the count of a completed epoch.
+template <int MODEL, bool ADAM>
+void launch_merge(mc_model* m, const GArgs& G) {
+    const bool one = G.shared_cnt <= 256;
+    const unsigned grid = one ? 1u : (unsigned)(1 + (G.shared_cnt + 255) / 256);
+    hipLaunchKernelGGL((grad_merge_kernel<MODEL, ADAM>), dim3(grid), dim3(256), 0, m->stream, G);
+    if (G.end_epoch && !one) hipLaunchKernelGGL(advance_epoch_kernel, dim3(1), dim3(64), 0, m->stream, G.steps);
+}
+
 template <int MODEL, bool ADAM>
 void launch_grad_t(mc_model* m, const GArgs& G0, int batch) {
     const size_t b = batch < 0 ? (size_t)m->n_batches : (size_t)batch;
@@ -725,19 +834,17 @@ void launch_grad_t(mc_model* m, const GArgs& G0, int batch) {
     Gb.shared_off = m->shared_off[b];
     Gb.shared_cnt = m->shared_cnt[b];
     const GArgs& G = Gb;
-    // Few items (a small minibatch): 1024 lanes per item to fill the chip.
-    const bool wide = nw + ng < 4 * (int64_t)m->n_cu;
+    const bool wide = wide_items(m, nw + ng);
     if (nw > 0) {
         if (wide) launch_items<MODEL, true, ADAM, 1024>(m, G, nw, m->win_off[b], grad_lds_bytes(m));
-        else launch_items<MODEL, true, ADAM, 256>(m, G, nw, m->win_off[b], grad_lds_bytes(m));
+        else launch_items<MODEL, true, ADAM, 512>(m, G, nw, m->win_off[b], grad_lds_bytes(m));
     }
     if (ng > 0) {
         if (wide) launch_items<MODEL, false, ADAM, 1024>(m, G, ng, m->glob_off[b], 0);
-        else launch_items<MODEL, false, ADAM, 256>(m, G, ng, m->glob_off[b], 0);
+        else launch_items<MODEL, false, ADAM, 512>(m, G, ng, m->glob_off[b], 0);
     }
-    const unsigned grid = (unsigned)(1 + (Gb.shared_cnt + 255) / 256);
-    hipLaunchKernelGGL((grad_merge_kernel<MODEL, ADAM>), dim3(grid), dim3(256), 0, m->stream, Gb);
-    if (ADAM && batch == m->n_batches - 1) hipLaunchKernelGGL(advance_epoch_kernel, dim3(1), dim3(64), 0, m->stream, G.steps);
+    Gb.end_epoch = ADAM && batch == m->n_batches - 1;
+    launch_merge<MODEL, ADAM>(m, Gb);
 }
 
 // One Adam step of an epoch replayed from a graph: the step of batch b also
@@ -780,10 +887,10 @@ void launch_fused_step_t(mc_model* m, int b) {
         }
         const size_t bi = (size_t)b;
         const int64_t nw = m->win_cnt[bi], ng = m->glob_cnt[bi];
-        const bool wide = nw + ng < 4 * (int64_t)m->n_cu;
+        const bool wide = wide_items(m, nw + ng);
         if (nw > 0) {
             if (wide) launch_items<MODEL, true, true, 1024>(m, G, nw, m->win_off[bi], grad_lds_bytes(m));
-            else launch_items<MODEL, true, true, 256>(m, G, nw, m->win_off[bi], grad_lds_bytes(m));
+            else launch_items<MODEL, true, true, 512>(m, G, nw, m->win_off[bi], grad_lds_bytes(m));
         }
         if (ng > 0) {
             // A second launch of the same step: the finalisation is done and
@@ -793,7 +900,7 @@ void launch_fused_step_t(mc_model* m, int b) {
                 G.sh_val = G.wr_val;
             }
             if (wide) launch_items<MODEL, false, true, 1024>(m, G, ng, m->glob_off[bi], 0);
-            else launch_items<MODEL, false, true, 256>(m, G, ng, m->glob_off[bi], 0);
+            else launch_items<MODEL, false, true, 512>(m, G, ng, m->glob_off[bi], 0);
         }
         return;
     }
@@ -808,9 +915,8 @@ void launch_fused_step_t(mc_model* m, int b) {
     G.sh_val = rd[3];
     G.sh_acc = m->d_gsh + (size_t)((B - 1) % 3) * kShAccSlot;
     G.zero_acc = m->d_gsh;
-    const unsigned grid = (unsigned)(1 + (G.shared_cnt + 255) / 256);
-    hipLaunchKernelGGL((grad_merge_kernel<MODEL, true>), dim3(grid), dim3(256), 0, m->stream, G);
-    hipLaunchKernelGGL(advance_epoch_kernel, dim3(1), dim3(64), 0, m->stream, G.steps);
+    G.end_epoch = 1;
+    launch_merge<MODEL, true>(m, G);
 }
 
 mc_status launch_fused_step(mc_model* m, int b) {

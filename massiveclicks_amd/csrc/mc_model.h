@@ -94,7 +94,7 @@ struct mc_model {
     std::vector<void*> allocations;
     // Pinned host chunks of stage_cap bytes through which results leave the
     // device (and the sessions of host-array evaluations enter it), one
-    // allocation made by the first call that needs them.
+    // allocation, made for the tables at init and grown by larger calls.
     char* stage[mc::kStages] = {};
     size_t stage_cap = 0;
     hipEvent_t stage_ev[mc::kStages] = {};

@@ -84,3 +84,27 @@ def test_queries_wider_than_the_item_window(model, pool, sizes, uneven):
     train, n_qd = sessions(sizes, pool, pool, uneven)
     print(f"case pool={pool} model={model} uneven={uneven} n_qd={n_qd}", flush=True)
     check(model, train, n_qd)
+
+
+@pytest.mark.parametrize("uneven", [False, True], ids=["ten", "uneven"])
+@pytest.mark.parametrize("model", list(IDS), ids=IDS.get)
+def test_gradient_does_not_depend_on_the_shape(model, uneven):
+    """Few wide items (1024 lanes), many (512 lanes), sliced queries and wide
+    queries give the same per-query gradient bit for bit (integer sums of the
+    same terms) and the same shared one up to the rounding of FP32 lane sums
+    (1e-6 of the sum of its terms, bounded here by the sessions' ranks)."""
+    train, n_qd = sessions([900, 3, 70] + [11] * 2500 + [1500], 400, 7, uneven)
+    got = []
+    for opts in ({}, {"item_sessions": 64}, {"item_sessions": 20000, "item_window": 1280}, {"packed": False}):
+        print(f"case gradient-shape model={model} uneven={uneven} {opts}", flush=True)
+        with ClickModel(model, **opts) as cm:
+            cm.init_parameters(train, n_qd)
+            cm.em(2)
+            ll, grads = cm.loglik_gradient()
+            got.append((ll, grads, cm.layout_info()["n_items"]))
+    assert max(g[2] for g in got) > 3 * 256 / 2 > min(g[2] for g in got)   # both sides of the lanes' rule
+    for ll, grads, _ in got[1:]:
+        assert ll == pytest.approx(got[0][0], rel=1e-6)
+        for t, g in enumerate(grads[:-1]):
+            np.testing.assert_allclose(g, got[0][1][t], rtol=2e-6, atol=2e-6)
+        np.testing.assert_allclose(grads[-1], got[0][1][-1], rtol=1e-6, atol=1e-6 * 10 * len(train))
