@@ -602,6 +602,37 @@ __global__ void fill_kernel(float* p, float v, int64_t n) {
     if (i < n) p[i] = v;
 }
 
+// reset_parameters in one launch: every per-qd entry and the shared table
+// (the last workgroup) to (1, 2), value 1/2.
+struct ResetArgs {
+    float *val[2], *num[2];
+    float *sh_val, *sh_num, *sh_den;
+    int64_t n_qd;
+    int32_t T, K;
+};
+__global__ void __launch_bounds__(256) reset_kernel(ResetArgs R) {
+    if (blockIdx.x == gridDim.x - 1) {
+        if ((int)threadIdx.x < R.K) {
+            R.sh_val[threadIdx.x] = 0.5f;
+            R.sh_num[threadIdx.x] = 1.f;
+            R.sh_den[threadIdx.x] = 2.f;
+        }
+        return;
+    }
+    const int64_t i = 4 * ((int64_t)blockIdx.x * blockDim.x + threadIdx.x);
+    for (int t = 0; t < R.T; t++) {
+        if (i + 4 <= R.n_qd) {
+            *reinterpret_cast<float4*>(R.val[t] + i) = make_float4(0.5f, 0.5f, 0.5f, 0.5f);
+            *reinterpret_cast<float4*>(R.num[t] + i) = make_float4(1.f, 1.f, 1.f, 1.f);
+        } else {
+            for (int64_t j = i; j < R.n_qd; j++) {
+                R.val[t][j] = 0.5f;
+                R.num[t][j] = 1.f;
+            }
+        }
+    }
+}
+
 }  // namespace mc
 
 // ===========================================================================
@@ -1363,15 +1394,21 @@ mc_status mc_set_parameters(mc_model* m, int t, const float* num, const float* d
 mc_status mc_reset_parameters(mc_model* m) {
     MC_REQUIRE(m && m->initialized, "model not initialised");
     MC_HIP(hipSetDevice(m->device));
-    for (int t = 0; t < m->T; t++) {
-        MC_TRY(fill(m, m->d_val[m->cur][t], 0.5f, m->n_qd));
-        MC_TRY(fill(m, m->d_num[m->cur][t], 1.f, m->n_qd));
-        m->den_state[t] = 0;
+    ResetArgs R;
+    for (int t = 0; t < 2; t++) {
+        R.val[t] = m->d_val[m->cur][t < m->T ? t : 0];
+        R.num[t] = m->d_num[m->cur][t < m->T ? t : 0];
     }
-    MC_TRY(fill(m, m->d_sh_val[m->cur], 0.5f, m->K));
-    MC_TRY(fill(m, m->d_sh_num[m->cur], 1.f, m->K));
-    MC_TRY(fill(m, m->d_sh_den[m->cur], 2.f, m->K));
+    R.sh_val = m->d_sh_val[m->cur];
+    R.sh_num = m->d_sh_num[m->cur];
+    R.sh_den = m->d_sh_den[m->cur];
+    R.n_qd = m->n_qd;
+    R.T = m->T;
+    R.K = m->K;
+    hipLaunchKernelGGL(reset_kernel, dim3((unsigned)((m->n_qd + 1023) / 1024 + 1)), dim3(256), 0, m->stream, R);
+    MC_HIP(hipGetLastError());
     MC_HIP(hipStreamSynchronize(m->stream));
+    for (int t = 0; t < m->T; t++) m->den_state[t] = 0;
     m->estep_pending = false;
     return MC_OK;
 }

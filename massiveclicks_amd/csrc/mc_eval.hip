@@ -306,12 +306,6 @@ __device__ __forceinline__ void eval_session(const EvalArgs& E, int L, const flo
     }
 }
 
-__device__ __forceinline__ double wave_sum_d(double v) {
-#pragma unroll
-    for (int off = 32; off >= 1; off >>= 1) v += __shfl_xor(v, off, 64);
-    return v;
-}
-
 // One session per lane, grid-stride: in every pass a wavefront takes 64
 // consecutive sessions.  Per-block FP64 partials of the 21 sums; the per-rank
 // session counts come from wavefront ballots (uniform values, no vector
@@ -413,10 +407,10 @@ __global__ void __launch_bounds__(256) eval_kernel(EvalArgs E) {
     if (OUT == kOutProb) return;
 #pragma unroll
     for (int k = 0; k < 11; k++) {
-        double w = wave_sum_d((double)v[k]);
-        if ((tid & 63) == 0) red[k][tid >> 6] = w;
+        const double w = wave_sum_last((double)v[k]);
+        if (lane == 63) red[k][tid >> 6] = w;
     }
-    if ((tid & 63) == 0)
+    if (lane == 0)   // the lane that took part in every pass
 #pragma unroll
         for (int r = 0; r < kL; r++) red[11 + r][tid >> 6] = (double)cnt[r];
     __syncthreads();

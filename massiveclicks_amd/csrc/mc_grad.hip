@@ -306,12 +306,6 @@ __device__ __forceinline__ float entry_gradient(int t, double sum, int2 oc, floa
     return (float)g;
 }
 
-__device__ __forceinline__ double wave_sum_f64(double v) {
-#pragma unroll
-    for (int off = 32; off >= 1; off >>= 1) v += __shfl_xor(v, off, 64);
-    return v;
-}
-
 // Merge work of grad_merge_kernel.
 __device__ __forceinline__ unsigned long long load_sum(const unsigned long long* p) { return *p; }
 // The sum of the kShParts copies of shared-table entry p[0].
@@ -523,8 +517,8 @@ __global__ void __launch_bounds__(NT) grad_item_kernel(GArgs G, int64_t list_off
         }
     }
     if (!ADAM) {
-        const double lw = wave_sum_f64((double)ll);
-        if (lane == 0) lred[wave] = lw;
+        const double lw = wave_sum_last((double)ll);
+        if (lane == 63) lred[wave] = lw;
     }
     __syncthreads();
     if constexpr (lslots) {   // eight lanes add up each slot's copies
@@ -730,6 +724,7 @@ mc_status ensure_grad_buffers(mc_model* m) {
     MC_HIP(hipMemcpy(m->d_sh_prior, prior.data(), prior.size() * 8, hipMemcpyHostToDevice));
     MC_HIP(hipDeviceGetAttribute(&m->n_cu, hipDeviceAttributeMultiprocessorCount, m->device));
     m->grad_ready = true;
+    m->grad_cleared = false;
     return MC_OK;
 }
 
@@ -1019,8 +1014,13 @@ mc_status mc_loglik_gradient(mc_model* m, int batch, double* loglik, float* cons
     MC_REQUIRE(batch >= -1 && batch < m->n_batches, "batch out of range");
     MC_HIP(hipSetDevice(m->device));
     MC_TRY(ensure_grad_buffers(m));
-    for (int t = 0; t < m->T; t++) MC_TRY(fill(m, m->d_grad[t], 0.f, m->n_qd));
-    MC_TRY(fill(m, (float*)m->d_ll_part, 0.f, 2 * (int64_t)m->n_items));
+    // The gradient of every session writes every entry a session shows and
+    // every item's log-likelihood; a minibatch's writes its own, over zeros.
+    if (batch >= 0 || !m->grad_cleared) {
+        for (int t = 0; t < m->T; t++) MC_TRY(fill(m, m->d_grad[t], 0.f, m->n_qd));
+        MC_TRY(fill(m, (float*)m->d_ll_part, 0.f, 2 * (int64_t)m->n_items));
+        m->grad_cleared = true;   // entries that no session shows stay 0
+    }
     MC_TRY(launch_grad(m, batch, false));
     if (loglik) {
         std::vector<double> part((size_t)m->n_items);

@@ -357,18 +357,9 @@ __device__ __forceinline__ void pbm_session(const int (&pv)[kL], int L, uint32_t
     }
 }
 
-// Examination slot of each rank for the UBM: r(r+1)/2 + prev[r], prev = 9
-// when no earlier click (ubm.cu:201, search.cu:184-198).
-__device__ __forceinline__ void ubm_slots(uint32_t mm, int (&slot)[kL]) {
-#pragma unroll
-    for (int r = 0; r < kL; r++) {
-        uint32_t before = mm & ((1u << r) - 1u);
-        int prev = before ? 31 - __builtin_clz(before) : kL - 1;
-        slot[r] = r * (r + 1) / 2 + prev;
-    }
-}
-
-// UBM E-step, ubm.cu:185-223.  The "no earlier click" slot of a rank can
+// UBM E-step, ubm.cu:185-223.  The examination slot of rank r is
+// r(r+1)/2 + prev, prev = 9 when there is no earlier click (ubm.cu:201,
+// search.cu:184-198).  The "no earlier click" slot of a rank can
 // coincide with a later rank's slot in the same session (e.g. no click
 // before rank 2 -> slot 12; click at rank 2 -> rank 4 uses slot 10 + 2 = 12);
 // the reference writes tmp[slot][session] in rank order, so only the last
@@ -774,13 +765,6 @@ __device__ __forceinline__ void decode_packed(PackedSession v, uint32_t& m, int&
     for (int r = 0; r < kL; r++) pv[r] = base + (int)((v[r >> 2] >> (8 * (r & 3))) & 0xffu);
 }
 
-// Wave-level sum of a 64-bit integer (wave64).
-__device__ __forceinline__ long long wave_sum(long long v) {
-#pragma unroll
-    for (int off = 32; off >= 1; off >>= 1) v += __shfl_xor(v, off, 64);
-    return v;
-}
-
 // Sum over the wavefront by DPP row shifts and broadcasts; valid in lane 63.
 template <int CTRL, int ROWS>
 __device__ __forceinline__ long long dpp_add(long long v) {
@@ -788,7 +772,17 @@ __device__ __forceinline__ long long dpp_add(long long v) {
     const int hi = __builtin_amdgcn_update_dpp(0, (int)(uint32_t)((unsigned long long)v >> 32), CTRL, ROWS, 0xf, true);
     return v + (long long)(((unsigned long long)(uint32_t)hi << 32) | (uint32_t)lo);
 }
-__device__ __forceinline__ long long wave_sum_last(long long v) {
+// (Cross-lane permutes through LDS instead: 12 instructions of LDS latency per
+// sum, 1.5 us of a 10 us evaluation kernel with its eleven sums.)
+template <int CTRL, int ROWS>
+__device__ __forceinline__ double dpp_add(double v) {
+    const long long b = __double_as_longlong(v);
+    const int lo = __builtin_amdgcn_update_dpp(0, (int)(uint32_t)b, CTRL, ROWS, 0xf, true);
+    const int hi = __builtin_amdgcn_update_dpp(0, (int)(uint32_t)((unsigned long long)b >> 32), CTRL, ROWS, 0xf, true);
+    return v + __longlong_as_double((long long)(((unsigned long long)(uint32_t)hi << 32) | (uint32_t)lo));
+}
+template <class V>
+__device__ __forceinline__ V wave_sum_last(V v) {
     v = dpp_add<0x111, 0xf>(v);   // row_shr:1
     v = dpp_add<0x112, 0xf>(v);   // row_shr:2
     v = dpp_add<0x114, 0xf>(v);   // row_shr:4

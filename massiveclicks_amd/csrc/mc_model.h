@@ -107,6 +107,7 @@ struct mc_model {
     int32_t* d_lists = nullptr;
     std::vector<int64_t> win_off, win_cnt, glob_off, glob_cnt, shared_off, shared_cnt;
     bool grad_ready = false;
+    bool grad_cleared = false;                 // d_grad is 0 wherever no session writes it
     float* d_logit[2] = {nullptr, nullptr};    // per-qd logits
     float* d_am[2] = {nullptr, nullptr};       // Adam first moments
     float* d_av[2] = {nullptr, nullptr};       // Adam second moments

@@ -75,8 +75,9 @@ def test_shapes_chosen_by_size(model, sizes, uneven):
 
 @pytest.mark.parametrize("model", list(IDS), ids=IDS.get)
 @pytest.mark.parametrize("pool,sizes,uneven", [(1300, [400, 30, 5000], False), (1300, [3000, 1, 800], True),
-                                               (3400, [2500, 60, 9000], False), (7500, [6000, 300], False)],
-                         ids=["1300", "1300-uneven", "3400", "7500"])
+                                               (3250, [3000, 10], False), (3400, [2500, 60, 9000], False),
+                                               (6000, [5000, 20], False), (7500, [6000, 300], False)],
+                         ids=["1300", "1300-uneven", "3250", "3400", "6000", "7500"])
 def test_queries_wider_than_the_item_window(model, pool, sizes, uneven):
     """Queries of more than 1280 entries: a window of their own, whole or
     sliced, up to what two workgroups per CU can hold (3,328 entries for the
@@ -95,12 +96,18 @@ def test_gradient_does_not_depend_on_the_shape(model, uneven):
     (1e-6 of the sum of its terms, bounded here by the sessions' ranks)."""
     train, n_qd = sessions([900, 3, 70] + [11] * 2500 + [1500], 400, 7, uneven)
     got = []
-    for opts in ({}, {"item_sessions": 64}, {"item_sessions": 20000, "item_window": 1280}, {"packed": False}):
+    for opts in ({}, {"item_sessions": 64}, {"item_sessions": 20000, "item_window": 1280}, {"packed": False},
+                 {"batches": 3}):
         print(f"case gradient-shape model={model} uneven={uneven} {opts}", flush=True)
         with ClickModel(model, **opts) as cm:
-            cm.init_parameters(train, n_qd)
+            cm.init_parameters(train, n_qd + 9)   # nine entries that no session shows
             cm.em(2)
+            if "batches" in opts:   # a part's gradient must leave nothing behind
+                cm.loglik_gradient(1)
             ll, grads = cm.loglik_gradient()
+            again = cm.loglik_gradient()
+            assert ll == again[0] and all(np.array_equal(x, y) for x, y in zip(grads, again[1]))
+            assert not any(g[n_qd:].any() for g in grads[:-1])
             got.append((ll, grads, cm.layout_info()["n_items"]))
     assert max(g[2] for g in got) > 3 * 256 / 2 > min(g[2] for g in got)   # both sides of the lanes' rule
     for ll, grads, _ in got[1:]:
