@@ -346,33 +346,34 @@ __device__ __forceinline__ void add_shared_sums(const KArgs& A, int item, const 
     }
 }
 
-// The same for the UBM's examination slots in LDS: the lanes first add their
-// "no earlier click" sums (registers) to their copy of the slots, then eight
-// lanes add up each slot's copies.
-template <int KACC, int NWMAX>
+// The same through LDS slots (fixed-point window paths): every lane adds its
+// sums to its copy of the slots, then eight lanes add up each slot's copies.
+// The UBM's lanes hold only the rows' "no earlier click" sums, its sessions
+// add to the other slots themselves.  One LDS atomic per sum and wavefront:
+// wavefront sums by DPP take about 24 VALU instructions per sum instead, a
+// tenth of the launch (per iteration, with DPP / with slots: 2M CCM sessions
+// 32.7 / 28.8 us, 8M PBM 62.4 / 56.1, 8M DBN 80.0 / 77.9).
+template <int MODEL>
 __device__ __forceinline__ void add_shared_slots(const KArgs& A, int item, const float (&acc)[55], unsigned long long* slots,
-                                                 long long (&red)[KACC][NWMAX], int tid, int nthr) {
-    unsigned long long* mine = slots + (tid & (kUbmCopies - 1));
+                                                 int tid, int nthr) {
+    constexpr int KACC = Shape<MODEL>::KACC;
+    unsigned long long* mine = slots + (tid & (kSlotCopies - 1));
 #pragma unroll
-    for (int r = 0; r < kL; r++) {
-        const int k = r * (r + 1) / 2 + kL - 1;
-        if (acc[k] != 0.f) atomicAdd(&mine[k * kUbmCopies], (unsigned long long)to_fix(acc[k]));
+    for (int r = 0; r < (MODEL == kUBM ? kL : KACC); r++) {
+        const int k = MODEL == kUBM ? r * (r + 1) / 2 + kL - 1 : r;
+        if (MODEL != kUBM || acc[k] != 0.f) atomicAdd(&mine[k * kSlotCopies], (unsigned long long)to_fix(acc[k]));
     }
     __syncthreads();
-    for (int q = tid; q < (kUbmSlots + 7) / 8 * 8 * 8; q += nthr) {
+    for (int q = tid; q < (KACC + 7) / 8 * 64; q += nthr) {
         const int k = q >> 3, c = q & 7;
         long long v = 0;
-        if (k < kUbmSlots)
+        if (k < KACC)
 #pragma unroll
-            for (int j = 0; j < kUbmCopies / 8; j++) v += (long long)slots[k * kUbmCopies + c + 8 * j];
-        v += __shfl_xor(v, 1, 64);
-        v += __shfl_xor(v, 2, 64);
-        v += __shfl_xor(v, 4, 64);
-        if (c == 0 && k < kUbmSlots) red[k][0] = v;
+            for (int j = 0; j < kSlotCopies / 8; j++) v += (long long)slots[k * kSlotCopies + c + 8 * j];
+        v = sum_of_eight(v);
+        if (c == 0 && v != 0)
+            atomicAdd(&A.sh_acc[(item & (A.sh_parts - 1)) * kShStride + k], (unsigned long long)v);
     }
-    __syncthreads();
-    if (tid < kUbmSlots && red[tid][0] != 0)
-        atomicAdd(&A.sh_acc[(item & (A.sh_parts - 1)) * kShStride + tid], (unsigned long long)red[tid][0]);
 }
 
 // Session paths, one kernel instantiation each (each gets its own register
@@ -400,7 +401,7 @@ __global__ void __launch_bounds__(512) em_item_kernel(KArgs A, int item_offset) 
     constexpr int KACC = Shape<MODEL>::KACC;
     extern __shared__ unsigned long long lds[];
     __shared__ float sh[K < 64 ? 64 : K];
-    __shared__ long long red[KACC][8];
+    __shared__ long long red[KACC][PATH == kPathLds || PATH == kPathPacked ? 1 : 8];
     __shared__ int last_one;
 
     const int item = item_offset + (int)blockIdx.x;
@@ -420,9 +421,10 @@ __global__ void __launch_bounds__(512) em_item_kernel(KArgs A, int item_offset) 
     const AccWindow<T> aw{lacc, Wmax, fixwin ? acc_copies_log2(W, Wmax) : 0};
     const int WS = W << aw.rsh;
     float* lval = fwin ? facc + T * W : (float*)(lds + T * Wmax);
-    // UBM examination slots in LDS after the window (fixed-point window path).
-    constexpr bool lslots = MODEL == kUBM && fixwin;
-    unsigned long long* slots = lds + ((size_t)T * Wmax * 12 + 7) / 8;
+    // Slots of the shared tables' sums: the UBM's after the window.
+    constexpr bool lslots = fixwin;
+    __shared__ unsigned long long few[lslots && MODEL != kUBM ? KACC * kSlotCopies : 1];
+    unsigned long long* slots = MODEL == kUBM ? lds + ((size_t)T * Wmax * 12 + 7) / 8 : few;
 
     // First session's loads go out before the window is staged.
     const Stream st = make_stream(A);
@@ -456,7 +458,7 @@ __global__ void __launch_bounds__(512) em_item_kernel(KArgs A, int item_offset) 
                         for (int t = 0; t < T; t++) lacc[aw.slot(t, i)] = 0ull;
                 }
                 if (lslots)
-                    for (int i = tid; i < kUbmSlots * kUbmCopies; i += nthr) slots[i] = 0ull;
+                    for (int i = tid; i < KACC * kSlotCopies; i += nthr) slots[i] = 0ull;
             }
 #pragma unroll
             for (int u = 0; u < U; u++) {
@@ -480,7 +482,7 @@ __global__ void __launch_bounds__(512) em_item_kernel(KArgs A, int item_offset) 
         EmitGlobalFloat em{A.tab[0].gaccf, A.tab[1].gaccf};
         run_item<MODEL, VARLEN, false>(st, it, gsrc, em, sh, acc, m0, L0, pv0);
     } else if (fixwin) {
-        EmitLds<T> em{aw, tid & ((1 << aw.rsh) - 1), slots + (tid & (kUbmCopies - 1))};
+        EmitLds<T> em{aw, tid & ((1 << aw.rsh) - 1), slots + (tid & (kSlotCopies - 1))};
         const SrcLds<T> lsrc{lval};
         if (packed) run_item_packed<MODEL, VARLEN>(st, it, lsrc, em, sh, acc, r0);
         else run_item<MODEL, VARLEN, true>(st, it, lsrc, em, sh, acc, m0, L0, pv0);
@@ -496,7 +498,7 @@ __global__ void __launch_bounds__(512) em_item_kernel(KArgs A, int item_offset) 
     }
 
     // Shared tables (also the barrier before the window is flushed).
-    if constexpr (lslots) add_shared_slots<KACC>(A, item, acc, slots, red, tid, nthr);
+    if constexpr (lslots) add_shared_slots<MODEL>(A, item, acc, slots, tid, nthr);
     else add_shared_sums<KACC>(A, item, acc, red, tid, nthr);
 
     if (fwin) {

@@ -130,7 +130,7 @@ struct EmitLdsSigned {             // as EmitLds: this lane's copies of the wind
     __device__ __forceinline__ void add(int t, int, int p, float x) {
         atomicAdd((unsigned long long*)(base[t] + (p << sh)), (unsigned long long)to_fix_signed(x));
     }
-    __device__ __forceinline__ void add_slot(int k, float x) { atomicAdd(&slots[k * kUbmCopies], to_fix_near(x)); }
+    __device__ __forceinline__ void add_slot(int k, float x) { atomicAdd(&slots[k * kSlotCopies], to_fix_near(x)); }
 };
 struct EmitGlobalSigned {
     static constexpr bool kSlotsInLds = false;
@@ -433,7 +433,7 @@ __global__ void __launch_bounds__(NT) grad_item_kernel(GArgs G, int64_t list_off
 #pragma unroll
                     for (int t = 0; t < T; t++) lds[aw.slot(t, i)] = 0ull;
                 if (lslots)
-                    for (int i = tid; i < kUbmSlots * kUbmCopies; i += NT) slots[i] = 0ull;
+                    for (int i = tid; i < K * kSlotCopies; i += NT) slots[i] = 0ull;
             }
 #pragma unroll
             for (int u = 0; u < U; u++) {
@@ -475,7 +475,7 @@ __global__ void __launch_bounds__(NT) grad_item_kernel(GArgs G, int64_t list_off
     {
         const SrcLds<T> lsrc{lval};
         const SrcGlobal gsrc{G.val[0], G.val[1]};
-        EmitLdsSigned<T> el{aw, tid & ((1 << aw.rsh) - 1), slots + (tid & (kUbmCopies - 1))};
+        EmitLdsSigned<T> el{aw, tid & ((1 << aw.rsh) - 1), slots + (tid & (kSlotCopies - 1))};
         EmitGlobalSigned eg{G.gacc[0], G.gacc[1]};
         if (packed) {
             for (int s = it.s0 + tid; s < it.s1; s += NT) {
@@ -503,11 +503,11 @@ __global__ void __launch_bounds__(NT) grad_item_kernel(GArgs G, int64_t list_off
     // accumulator and item.
     const int wave = tid >> 6, lane = tid & 63;
     if constexpr (lslots) {
-        unsigned long long* mine = slots + (tid & (kUbmCopies - 1));
+        unsigned long long* mine = slots + (tid & (kSlotCopies - 1));
 #pragma unroll
         for (int r = 0; r < kL; r++) {
             const int k = r * (r + 1) / 2 + kL - 1;
-            if (acc[k] != 0.f) atomicAdd(&mine[k * kUbmCopies], (unsigned long long)to_fix_signed(acc[k]));
+            if (acc[k] != 0.f) atomicAdd(&mine[k * kSlotCopies], (unsigned long long)to_fix_signed(acc[k]));
         }
     } else {
 #pragma unroll
@@ -522,16 +522,14 @@ __global__ void __launch_bounds__(NT) grad_item_kernel(GArgs G, int64_t list_off
     }
     __syncthreads();
     if constexpr (lslots) {   // eight lanes add up each slot's copies
-        for (int q = tid; q < 8 * ((kUbmSlots + 7) / 8 * 8); q += NT) {
+        for (int q = tid; q < 8 * ((K + 7) / 8 * 8); q += NT) {
             const int k = q >> 3, c = q & 7;
             long long v = 0;
-            if (k < kUbmSlots)
+            if (k < K)
 #pragma unroll
-                for (int j = 0; j < kUbmCopies / 8; j++) v += (long long)slots[k * kUbmCopies + c + 8 * j];
-            v += __shfl_xor(v, 1, 64);
-            v += __shfl_xor(v, 2, 64);
-            v += __shfl_xor(v, 4, 64);
-            if (c == 0 && k < kUbmSlots && v != 0)
+                for (int j = 0; j < kSlotCopies / 8; j++) v += (long long)slots[k * kSlotCopies + c + 8 * j];
+            v = sum_of_eight(v);
+            if (c == 0 && k < K && v != 0)
                 atomicAdd(&G.sh_acc[(blockIdx.x % kShParts) * kShAccStride + k], (unsigned long long)v);
         }
     }

@@ -235,19 +235,17 @@ __device__ __forceinline__ int acc_copies_log2(int W, int wstride) {
 // t for the entry p shown at rank r of the current session; add_wide takes
 // any non-negative x (the CCM's last-click attractiveness term can exceed 1;
 // the last-click terms, once per session, always take it).
-// UBM examination counts of a workgroup in LDS: kUbmSlots fixed-point
-// accumulators, each in kUbmCopies copies; lane l adds into copy
-// l mod kUbmCopies, so the lanes of one instruction never share an address
-// with more than one other lane.  Laid out [slot][copy].
-constexpr int kUbmSlots = 55;
-constexpr int kUbmCopies = 32;
-constexpr size_t kUbmSlotBytes = (size_t)kUbmSlots * kUbmCopies * 8;
+// Shared-table sums of a workgroup in LDS: fixed-point slots in kSlotCopies
+// copies each, laid out [slot][copy]; lane l adds into copy l mod kSlotCopies,
+// so the lanes of one instruction never share an address with more than one
+// other lane.
+constexpr int kSlotCopies = 32;
 
 template <int T>
 struct EmitLds {            // fixed-point LDS window, relative indices
     char* base[T];             // this lane's copy of entry 0 of each table: &acc[slot(t, copy)]
     int sh;                    // rsh + 3: entry p's copies start p << sh bytes further
-    unsigned long long* slots; // UBM: this lane's copy of the examination slots (stride kUbmCopies)
+    unsigned long long* slots; // UBM: this lane's copy of the examination slots (stride kSlotCopies)
     static constexpr bool kSlotsInLds = true;
     __device__ __forceinline__ EmitLds(const AccWindow<T>& w, int copy, unsigned long long* lane_slots)
         : sh(w.rsh + 3), slots(lane_slots) {
@@ -262,7 +260,7 @@ struct EmitLds {            // fixed-point LDS window, relative indices
     __device__ __forceinline__ void add_wide(int t, int, int p, float x) {
         atomicAdd(at(t, p), (unsigned long long)to_fix(x));
     }
-    __device__ __forceinline__ void add_slot(int k, float x) { atomicAdd(&slots[k * kUbmCopies], to_fix_unit(x)); }
+    __device__ __forceinline__ void add_slot(int k, float x) { atomicAdd(&slots[k * kSlotCopies], to_fix_unit(x)); }
 };
 struct EmitGlobalFix {      // fixed-point global (item without a window)
     static constexpr bool kSlotsInLds = false;
@@ -662,13 +660,13 @@ template <> struct Shape<kDBN> { static constexpr int T = 2, K = 1, KACC = 2; };
 template <> struct Shape<kCCM> { static constexpr int T = 1, K = 3, KACC = 6; };
 
 // Dynamic LDS of a window launch of `width` entries: accumulators and staged
-// values (the float-atomic mode's are 8 bytes an entry), then the UBM's
-// examination slots.
+// values (the float-atomic mode's are 8 bytes an entry), then the UBM's slots
+// (the other models' few are static).
 inline size_t window_lds_bytes(int type, int reduce_mode, int width) {
     const size_t T = type == kDBN ? 2 : 1;
     if (reduce_mode != 0) return (size_t)width * T * 8;
     const size_t b = (size_t)width * T * 12;
-    return type == kUBM ? (b + 7) / 8 * 8 + kUbmSlotBytes : b;
+    return type == kUBM ? (b + 7) / 8 * 8 + (size_t)Shape<kUBM>::KACC * kSlotCopies * 8 : b;
 }
 
 // Buffer descriptors of the session stream: 32-bit offsets (no 64-bit
@@ -780,6 +778,12 @@ __device__ __forceinline__ double dpp_add(double v) {
     const int lo = __builtin_amdgcn_update_dpp(0, (int)(uint32_t)b, CTRL, ROWS, 0xf, true);
     const int hi = __builtin_amdgcn_update_dpp(0, (int)(uint32_t)((unsigned long long)b >> 32), CTRL, ROWS, 0xf, true);
     return v + __longlong_as_double((long long)(((unsigned long long)(uint32_t)hi << 32) | (uint32_t)lo));
+}
+// Sum of aligned groups of eight lanes, valid in all of them.
+__device__ __forceinline__ long long sum_of_eight(long long v) {
+    v = dpp_add<0xB1, 0xf>(v);    // quad_perm [1, 0, 3, 2]
+    v = dpp_add<0x4E, 0xf>(v);    // quad_perm [2, 3, 0, 1]
+    return dpp_add<0x141, 0xf>(v);   // row_half_mirror
 }
 template <class V>
 __device__ __forceinline__ V wave_sum_last(V v) {
