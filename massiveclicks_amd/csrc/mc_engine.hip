@@ -54,7 +54,8 @@ __device__ __forceinline__ void run_session_len(const int (&pv)[kL], uint32_t m,
         ubm_session(pv, LC, mm, src, em, sh, acc);
     } else if (MODEL == kDBN) {
         if (mm == 0) return;   // every count of a click-free session is a constant
-        // The gamma and tau sums go straight into the lane's accumulators.
+        // The gamma and tau sums go straight into the lane's accumulators
+        // (shared_sums gives them their factors at the end of the item).
         dbn_session<VARLEN>(pv, LC, mm, src, em, sh[0], acc[0], acc[1]);
     } else {
         if (mm == 0) return;
@@ -498,6 +499,7 @@ __global__ void __launch_bounds__(512) em_item_kernel(KArgs A, int item_offset) 
     }
 
     // Shared tables (also the barrier before the window is flushed).
+    shared_sums<MODEL>(sh, acc);
     if constexpr (lslots) add_shared_slots<MODEL>(A, item, acc, slots, tid, nthr);
     else add_shared_sums<KACC>(A, item, acc, red, tid, nthr);
 

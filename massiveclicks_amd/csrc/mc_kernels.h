@@ -456,22 +456,23 @@ __device__ __forceinline__ float pick10(const float (&v)[kL], int i) {
 //   E_{lcr+1} = g(1-s_lcr), E_{r+1} = E_r t_r / (1 - a_r E_r).
 template <bool VARLEN, class Src, class Emit>
 __device__ __forceinline__ void dbn_session(const int (&pv)[kL], int L, uint32_t mm, const Src& src, Emit& em,
-                                            float g, float& gn, float& gd) {
+                                            float g, float& sgt, float& sw) {
     // The chains are restructured algebra rather than the reference's
     // operation order, so multiply-adds may fuse here.
 #pragma clang fp contract(fast)
     const int lcr = last_click(mm);
     // Pass 1, ranks 0..L-1: exam[r] (compute_exm_car) and the no-click tail
-    // products V_k; only exam[r] for r > lcr and V_k for k < L - lcr are used.
+    // products times gamma, g V_k (G scaled likewise costs nothing); only
+    // exam[r] for r > lcr and V_k for k < L - lcr are used.
     // The examination factor t + g a (1 - s) equals g (1 - a s): with
     // ga = g a, one multiply-add gives it and one subtraction gives t.
-    float exam[kL], V[kL];
+    float exam[kL], gV[kL];
     {
-        float e = 1.f, v = 1.f, G = 1.f;
+        float e = 1.f, v = g, G = g;
 #pragma unroll
         for (int r = 0; r < kL; r++) {
             exam[r] = e;
-            V[r] = v;
+            gV[r] = v;
             if (!VARLEN || r < L) {
                 const float2 as = src.pair(pv[r]);
                 const float ga = g * as.x;
@@ -498,38 +499,41 @@ __device__ __forceinline__ void dbn_session(const int (&pv)[kL], int L, uint32_t
     // Pass 3, ranks lcr..L-1: satisfaction at the last click, gamma factors.
     // After the last click the conditional examination probability E
     // follows E_{r+1} = E_r g(1-a_r) / d2, d2 = 1 - a_r E_r, and the factor
-    // ratios of an unclicked rank are phi5/sum = g T E / d1 and
-    // (phi4+phi5)/sum = E (1-g+gT) / d1, d1 = 1 - g E (1-T).  Both divisions
-    // share one reciprocal q = 1/(d1 d2): 1/d1 = d2 q, 1/d2 = d1 q.  E <= g,
-    // so d1, d2 >= 1 - g >= 1e-6 (clamped gamma) and d1 d2 is a normal float.
+    // ratios of an unclicked rank are phi5/sum = g T w and
+    // (phi4+phi5)/sum = (1 - g + g T) w with w = E / d1, d1 = 1 - g E + g T E;
+    // at the last click the same with w = (1-s) / (phi4 + phi5 + s).  The
+    // lane adds up w and g T w; shared_sums turns them into the two counts.
+    // E <= g, so d1, d2 >= 1 - g >= 1e-6 (clamped gamma).  A reciprocal each
+    // (two VALU slots) costs less than one of d1 d2 and its three multiplies;
+    // with the weights and the separate loops below, per iteration: 8M
+    // sessions 77.5 -> 73.3 us, 500,000 15.2 -> 14.6.
     __asm__ volatile("" ::: "memory");
+    // One loop for the last click and one for the ranks after it: as arms of
+    // one branch they copy the sums at every rank.
     float E = 0.f;
 #pragma unroll
     for (int r = 0; r < kL; r++) {
-        if ((!VARLEN || r < L) && r >= lcr) {
-            float Tn;
-            if (VARLEN) Tn = (r + 1 < L) ? pick10(V, L - 1 - r) : 1.f;
-            else Tn = (r + 1 < kL) ? V[(kL - 1 - r) < 0 ? 0 : (kL - 1 - r)] : 1.f;
-            if (r == lcr) {
-                const float sv = src.get(1, pv[r]);
-                // At most 1 (g car <= 1), so the unit conversion applies.
-                em.add(1, r, pv[r], fdiv(sv, 1 - (1 - sv) * g * car));
-                const float phi4 = (1 - sv) * (1 - g);
-                const float phi5 = (1 - sv) * g * Tn;
-                const float inv = __builtin_amdgcn_rcpf(phi4 + phi5 + sv);
-                gn += phi5 * inv;
-                gd += (phi4 + phi5) * inv;
-                E = g * (1 - sv);
-            } else {
-                const float a = src.get(0, pv[r]);
-                const float d1 = 1 - g * E * (1 - Tn);
-                const float d2 = 1 - a * E;
-                const float q = __builtin_amdgcn_rcpf(d1 * d2);
-                const float w = E * (d2 * q);
-                gn += g * Tn * w;
-                gd += (1 - g + g * Tn) * w;
-                E = E * (g * (1 - a)) * (d1 * q);
-            }
+        if ((!VARLEN || r < L) && r == lcr) {
+            const float gT = VARLEN ? pick10(gV, L - 1 - r) : gV[kL - 1 - r];
+            const float sv = src.get(1, pv[r]);
+            const float ns = 1 - sv;
+            // At most 1 (g car <= 1), so the unit conversion applies.
+            em.add(1, r, pv[r], fdiv(sv, 1 - ns * g * car));
+            const float w = ns * __builtin_amdgcn_rcpf(ns * ((1 - g) + gT) + sv);
+            sw += w;
+            sgt += gT * w;
+            E = g * ns;
+        }
+    }
+#pragma unroll
+    for (int r = 1; r < kL; r++) {
+        if ((!VARLEN || r < L) && r > lcr) {
+            const float gT = VARLEN ? pick10(gV, L - 1 - r) : gV[kL - 1 - r];
+            const float a = src.get(0, pv[r]);
+            const float w = E * __builtin_amdgcn_rcpf((1 - g * E) + gT * E);
+            sw += w;
+            sgt += gT * w;
+            E = E * (g - g * a) * __builtin_amdgcn_rcpf(1 - a * E);
         }
     }
 }
@@ -589,61 +593,71 @@ __device__ __forceinline__ void ccm_session(const int (&pv)[kL], int L, uint32_t
         }
     }
     // Pass 3, ranks 0..L-1: tau2/tau3 posteriors of earlier clicks, the last
-    // click, and the tau1 factors after it.
+    // click, and the tau1 factors after it.  With T the tail product, every
+    // factor of tau_i is (tau_i T w, ((1 - tau_i) + tau_i T) w) for a weight w:
+    // after the last click w = E / d1, d1 = 1 - tau1 E + tau1 T E; at it
+    // w = (1-a) / sum for tau2 and a / sum for tau3; an earlier click counts
+    // tau_i w to both, so it adds to the first sum only.  The lane adds up
+    // T w and w per table; shared_sums applies the factors.  Per iteration,
+    // with the factors per rank and one branch for the three kinds of rank:
+    // 8M sessions 74.3 us, 2M 29.2; like this 68.5 and 27.6.
     __asm__ volatile("" ::: "memory");
-    float ex = 0.f;
+    // Three loops, one per kind of rank: as arms of one branch they copy the
+    // sums at every rank.
+    const uint32_t earlier = mm ^ (1u << lcr);
+#pragma unroll
+    for (int r = 0; r < kL - 1; r++) {
+        if ((!VARLEN || r < L) && ((earlier >> r) & 1u)) {
+            const float a = src.get(0, pv[r]);
+            const float na = 1 - a;
+            const float inv = __builtin_amdgcn_rcpf(na * t2 + a * t3);
+            ta[2] += na * inv;
+            ta[4] += a * inv;
+        }
+    }
+    float E = 0.f;
 #pragma unroll
     for (int r = 0; r < kL; r++) {
-        if (VARLEN && r >= L) continue;
-        const bool clicked = (mm >> r) & 1u;
-        if (r < lcr) {
-            if (clicked) {
-                const float a = src.get(0, pv[r]);
-                const float w2 = (1 - a) * t2;
-                const float w3 = a * t3;
-                const float inv = __builtin_amdgcn_rcpf(w2 + w3);
-                const float x = w2 * inv;
-                const float y = w3 * inv;
-                ta[2] += x; ta[3] += x;
-                ta[4] += y; ta[5] += y;
-            }
-            continue;
+        if ((!VARLEN || r < L) && r == lcr) {
+            const float Tn = VARLEN ? pick10(V, L - 1 - r) : V[kL - 1 - r];
+            const float a = src.get(0, pv[r]);
+            const float na = 1 - a;
+            E = t2 * na + t3 * a;
+            em.add_wide(0, r, pv[r], fdiv(a, 1 - E * car));
+            const float inv = __builtin_amdgcn_rcpf((na * (1 - t2) + a * (1 - t3)) + E * Tn);
+            const float w2 = na * inv;
+            const float w3 = a * inv;
+            ta[2] += Tn * w2;
+            ta[3] += w2;
+            ta[4] += Tn * w3;
+            ta[5] += w3;
         }
-        const float a = src.get(0, pv[r]);
-        float Tn;
-        if (VARLEN) Tn = (r + 1 < L) ? pick10(V, L - 1 - r) : 1.f;
-        else Tn = (r + 1 < kL) ? V[(kL - 1 - r) < 0 ? 0 : (kL - 1 - r)] : 1.f;
-        if (r == lcr) {
-            em.add_wide(0, r, pv[r], fdiv(a, 1 - (t2 * (1 - a) + t3 * a) * car));
-            const float phi4 = (1 - a) * (1 - t2);
-            const float phi5 = (1 - a) * t2 * Tn;
-            const float phi6 = a * (1 - t3);
-            const float phi7 = a * t3 * Tn;
-            const float inv = __builtin_amdgcn_rcpf(phi4 + phi5 + phi6 + phi7);
-            const float n2 = phi5 * inv;
-            const float n3 = phi7 * inv;
-            ta[2] += n2;
-            ta[3] += n2 + phi4 * inv;
-            ta[4] += n3;
-            ta[5] += n3 + phi6 * inv;
-            ex = t2 * (1 - a) + t3 * a;
-        } else {
-            // The factor sum d1 and the examination update's denominator d2
-            // share one reciprocal: q = 1/(d1 d2), 1/d1 = d2 q, 1/d2 = d1 q.
-            // Both are at least 1e-6 (clamped parameters), so d1 d2 is a
-            // normal float.
-            const float E = ex;
-            const float phi0 = 1 - E;
-            const float phi4 = (1 - t1) * E;
-            const float phi5 = t1 * Tn * E;
-            const float d1 = phi0 + phi4 + phi5;
-            const float d2 = 1 - a * E;
-            const float q = __builtin_amdgcn_rcpf(d1 * d2);
-            const float inv = d2 * q;
-            const float n1 = phi5 * inv;
-            ta[0] += n1;
-            ta[1] += n1 + phi4 * inv;
-            ex = E * (t1 * (1 - a)) * (d1 * q);
+    }
+#pragma unroll
+    for (int r = 1; r < kL; r++) {
+        if ((!VARLEN || r < L) && r > lcr) {
+            // d1, d2 >= 1e-6 (clamped parameters).
+            const float Tn = VARLEN ? pick10(V, L - 1 - r) : V[kL - 1 - r];
+            const float a = src.get(0, pv[r]);
+            const float w = E * __builtin_amdgcn_rcpf((1 - t1 * E) + t1 * E * Tn);
+            ta[0] += Tn * w;
+            ta[1] += w;
+            E = E * (t1 - t1 * a) * __builtin_amdgcn_rcpf(1 - a * E);
+        }
+    }
+}
+
+// The lane's sums of T w and w (DBN: g T w and w) into the counts of the
+// shared tables, once per work item.
+template <int MODEL>
+__device__ __forceinline__ void shared_sums(const float* sh, float (&acc)[55]) {
+    if constexpr (MODEL == kDBN) {
+        acc[1] = acc[0] + (1 - sh[0]) * acc[1];
+    } else if constexpr (MODEL == kCCM) {
+#pragma unroll
+        for (int i = 0; i < 3; i++) {
+            acc[2 * i] *= sh[i];
+            acc[2 * i + 1] = acc[2 * i] + (1 - sh[i]) * acc[2 * i + 1];
         }
     }
 }
