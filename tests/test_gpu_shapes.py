@@ -21,14 +21,17 @@ IDS = {PBM: "PBM", UBM: "UBM", DBN: "DBN", CCM: "CCM"}
 
 def sessions(sizes, pool, seed, uneven=False):
     """Query-grouped sessions: `sizes[q]` sessions of query q, ten of its
-    `pool` documents each; pair indices are contiguous per query."""
+    `pool` documents each; pair indices are contiguous per query.  `uneven`:
+    random lengths, or the lengths."""
     rng = np.random.default_rng(seed)
     query = np.repeat(np.arange(len(sizes), dtype=np.int32), sizes)
     n = len(query)
     slot = np.argsort(rng.random((n, pool), np.float32), axis=1)[:, :10]
     raw = query[:, None].astype(np.int64) * pool + slot
-    length = rng.integers(1, 11, n).astype(np.uint8) if uneven else None
-    shown = np.arange(10)[None, :] < (length[:, None] if uneven else np.full((n, 1), 10))
+    length = None
+    if uneven is not False:
+        length = rng.integers(1, 11, n).astype(np.uint8) if uneven is True else np.asarray(uneven, np.uint8)
+    shown = np.arange(10)[None, :] < (np.full((n, 1), 10) if length is None else length[:, None])
     used, inv = np.unique(raw[shown], return_inverse=True)
     pidx = np.full((n, 10), -1, np.int32)
     pidx[shown] = inv
@@ -115,3 +118,15 @@ def test_gradient_does_not_depend_on_the_shape(model, uneven):
         for t, g in enumerate(grads[:-1]):
             np.testing.assert_allclose(g, got[0][1][t], rtol=2e-6, atol=2e-6)
         np.testing.assert_allclose(grads[-1], got[0][1][-1], rtol=1e-6, atol=1e-6 * 10 * len(train))
+
+
+@pytest.mark.parametrize("model", list(IDS), ids=IDS.get)
+@pytest.mark.parametrize("packed", [True, False], ids=["packed", "rank-major"])
+@pytest.mark.parametrize("lengths", [[1], [10] * 64, [3] * 70, [10] * 63 + [1], list(range(1, 11)) * 7,
+                                     sorted(list(range(1, 11)) * 64)],
+                         ids=["one", "ten", "three", "odd-one", "mixed", "blocks"])
+def test_lengths_of_a_wavefront(model, packed, lengths):
+    """Wavefronts of one length, of one length but for a lane, and of all."""
+    train, n_qd = sessions([len(lengths)], 30, seed=len(lengths), uneven=lengths)
+    print(f"case wavefront lengths model={IDS[model]} n={len(lengths)} packed={packed}", flush=True)
+    check(model, train, n_qd, packed=packed)
