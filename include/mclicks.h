@@ -45,9 +45,10 @@ enum {
     /* Target sessions per workgroup work item (default: chosen for the
      * training set, 256 to 16384; 8192 in the float-atomic mode). */
     MC_OPT_ITEM_SESSIONS = 1,
-    /* Per-qd accumulator window per work item, in entries (default 1280,
-     * with a window of its own for a query of more entries, as far as LDS
-     * goes; when set, such queries use global atomics). */
+    /* Per-qd accumulator window per work item, in entries (default 1280, or
+     * up to 2048 for a million sessions and more, with a window of its own
+     * for a query of more entries, as far as LDS goes; when set, such queries
+     * use global atomics). */
     MC_OPT_ITEM_WINDOW = 2,
     /* 1 = reorder sessions inside each work item by length, then last-click
      * rank, so that wavefronts run uniform chains (default 1). */

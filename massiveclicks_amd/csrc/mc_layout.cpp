@@ -31,6 +31,7 @@ void choose_shape(mc_model* m, int64_t n, bool uneven) {
     if (m->reduce_mode != MC_REDUCE_SEGMENTED) {
         if (!m->block_set) m->block = 256;
         if (!m->item_sessions_set) m->item_sessions = 8192;
+        if (!m->item_window_set) m->item_window = 1280;
         return;
     }
     // PBM and CCM windows (15 KB of LDS) let eight 256-lane workgroups onto a
@@ -50,6 +51,20 @@ void choose_shape(mc_model* m, int64_t n, bool uneven) {
     if (!m->item_sessions_set) {
         const int64_t per = m->block >= 512 ? (uneven ? 384 : n < 1000000 ? 256 : 512) : (uneven ? 512 : 1024);
         m->item_sessions = (int)std::min<int64_t>(16384, std::max<int64_t>(256, n / per));
+    }
+    // The window of a large set is the widest that leaves a CU's 32 wavefronts
+    // their share of its 160 KB of LDS (24 bytes an entry for the DBN, else
+    // 12, the UBM's slots 14 KB): the rare queries then fill fewer items, each
+    // with its staging and counting.  Us per iteration with 1280 entries / so
+    // many: UBM 8M 81.5 / 71.4, 1M 19.8 / 18.3; DBN 8M 76.7 / 74.0, 1M 20.4 /
+    // 18.5, 2M 28.7 / 28.9; CCM 8M 71.0 / 70.5, 2M 28.2 / 26.9.  Small sets
+    // are better off with more items (500,000 DBN 14.4 / 14.1, 312,000 UBM
+    // 10.8 / 11.0), the PBM gains nothing (8M 56.6 / 56.3, 2M 23.2 / 23.6).
+    if (!m->item_window_set) {
+        m->item_window = 1280;
+        if (n >= 1000000 && m->block == 512 && m->type == MC_UBM) m->item_window = 2048;
+        if (n >= 1000000 && m->block == 512 && m->type == MC_DBN) m->item_window = 1600;
+        if (n >= 1000000 && m->block == 256 && m->type == MC_CCM) m->item_window = 1504;
     }
 }
 

@@ -92,7 +92,7 @@ extern "C" mc_status mc_autotune(int model_type, int device, int64_t n, const in
     for (int64_t s : {512, 1024, 2048, 4096, 8192, 16384})
         if ((st = attempt(MC_OPT_ITEM_SESSIONS, s)) != MC_OK) return st;
     if (best[MC_OPT_REDUCE_MODE] == MC_REDUCE_SEGMENTED) {
-        for (int64_t w : {512, 1024, 1280})
+        for (int64_t w : {512, 1024, 1280, 1600, 2048})
             if ((st = attempt(MC_OPT_ITEM_WINDOW, w)) != MC_OK) return st;
         // Lanes per work item.
         for (int64_t b : {256, 512})

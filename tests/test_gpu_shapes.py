@@ -130,3 +130,14 @@ def test_lengths_of_a_wavefront(model, packed, lengths):
     train, n_qd = sessions([len(lengths)], 30, seed=len(lengths), uneven=lengths)
     print(f"case wavefront lengths model={IDS[model]} n={len(lengths)} packed={packed}", flush=True)
     check(model, train, n_qd, packed=packed)
+
+
+@pytest.mark.parametrize("model,window,block", [(UBM, 2048, 512), (DBN, 1600, 512), (CCM, 1504, 256)],
+                         ids=["UBM", "DBN", "CCM"])
+@pytest.mark.parametrize("queries", [75, 103, 400])
+def test_windows_of_large_sets(model, window, block, queries):
+    """The item windows chosen for large sets: entries below, at and above
+    one window, and several windows."""
+    train, n_qd = sessions([2] * queries, 20, seed=queries)
+    print(f"case windows of large sets model={IDS[model]} entries={n_qd}", flush=True)
+    check(model, train, n_qd, item_window=window, block=block)
