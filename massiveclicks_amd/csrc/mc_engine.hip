@@ -1208,7 +1208,8 @@ mc_status mc_init_parameters(mc_model* m, int64_t n, const int32_t* query, const
         MC_TRY(fill(m, m->d_sh_den[b], 2.f, K));
     }
     m->den_state[T] = 0;
-    MC_TRY(stage_reserve(m, stage_chunk((size_t)n_qd * 4)));   // for the tables' readback
+    // For the tables' readback and evaluations of a few thousand host rows.
+    MC_TRY(stage_reserve(m, std::max(stage_chunk((size_t)n_qd * 4), (size_t)64 << 10)));
     MC_HIP(hipStreamSynchronize(m->stream));
     m->cur = 0;
     m->estep_pending = false;

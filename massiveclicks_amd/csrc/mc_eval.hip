@@ -577,12 +577,15 @@ mc_status evaluate_host_arrays(mc_model* m, int64_t n, const int32_t* pidx, cons
     const size_t a_p = place(row * chunk, true), a_c = place((size_t)kMaxSerp * chunk, true);
     const size_t a_l = place((size_t)chunk, len), a_lp = place(row * chunk, logp), a_fp = place(row * chunk, full);
     const size_t a_llh = place((size_t)chunk * 4, llh), a_pr = place(row * chunk, prob);
-    MC_TRY(stage_reserve(m, place(0, true)));
+    const size_t bytes = (place(0, true) + 255) / 256 * 256;
+    // One or two chunks in the model's pinned slots, which lie side by side.
+    MC_TRY(stage_reserve(m, (bytes * (size_t)std::min<int64_t>(n_chunks, 2) + kStages - 1) / kStages));
+    auto buffer = [&](int64_t k) { return m->stage[0] + (size_t)(k & 1) * bytes; };
     constexpr int64_t kMaxNb = kEvalChunk / 256;
     if (!m->d_eval_part) MC_TRY(dalloc(m, &m->d_eval_part, (size_t)(kMaxNb + 1) * 21 * 8));
     double* running = m->d_eval_part + kMaxNb * 21;
     auto copy_out = [&](int64_t k) -> mc_status {
-        const char* b = m->stage[k & 1];
+        const char* b = buffer(k);
         const size_t at = (size_t)(k * chunk), c = (size_t)std::min(chunk, n - k * chunk);
         MC_HIP(hipEventSynchronize(m->stage_ev[k & 1]));
         if (logp) std::memcpy(logp + at * kMaxSerp, b + a_lp, row * c);
@@ -592,7 +595,7 @@ mc_status evaluate_host_arrays(mc_model* m, int64_t n, const int32_t* pidx, cons
         return MC_OK;
     };
     auto enqueue = [&](int64_t k) -> mc_status {
-        char* b = m->stage[k & 1];
+        char* b = buffer(k);
         const size_t at = (size_t)(k * chunk), c = (size_t)std::min(chunk, n - k * chunk);
         std::memcpy(b + a_p, pidx + at * kMaxSerp, row * c);
         std::memcpy(b + a_c, clicks + at * kMaxSerp, (size_t)kMaxSerp * c);
