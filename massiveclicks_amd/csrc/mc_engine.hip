@@ -403,17 +403,19 @@ __device__ __forceinline__ void add_shared_slots(const KArgs& A, int item, const
 enum { kPathLds = 0, kPathGlobal = 1, kPathAtomic = 2, kPathDirect = 3, kPathLdsFloat = 4, kPathPacked = 5 };
 
 // E-step and in-item M-step of one work item (item index item_offset +
-// blockIdx.x).  Bound by the VALU on large sets (8M DBN sessions: 380
-// instructions per 64 sessions, about 70 of 82 us) and by the chain of load,
+// blockIdx.x).  Bound by the VALU on large sets (8M sessions, instructions at
+// four cycles of the launch: DBN 58 of 76 us, CCM 67 of 73), by the latency
+// of the rare queries' items on medium ones and by the chain of load,
 // session, flush and counter round trips on small ones (32,000 PBM sessions:
-// 5 us of 8, the launch gap included).  At 37-64 VGPRs the packed paths keep
-// 32 wavefronts on a CU, and the hardware hands each freed slot the next
+// 5 us of 7.4, the launch gap included).  At 37-64 VGPRs the packed paths
+// keep 32 wavefronts on a CU, and the hardware hands each freed slot the next
 // item: a persistent form with a fixed item list per workgroup held the next
-// item's window in 77-103 VGPRs and took 87 us on those 8M sessions.  Dynamic LDS (window path): width x T fixed-point
-// accumulators, then width x T staged values of theta_t (both interleaved per
-// entry).  kPathLdsFloat (float-atomic mode) pre-reduces in float LDS
-// accumulators and adds every window entry to global float accumulators,
-// which the merge kernel finalises.
+// item's window in 77-103 VGPRs and took 87 us on 8M DBN sessions where this,
+// with the same session code, took 82.  Dynamic LDS (window path): width x T
+// fixed-point accumulators (AccWindow), then width x T staged values of
+// theta_t, interleaved per entry, then the UBM's slots.  kPathLdsFloat (float-atomic mode) pre-reduces in
+// float LDS accumulators and adds every window entry to global float
+// accumulators, which the merge kernel finalises.
 template <int MODEL, bool VARLEN, int PATH>
 __global__ void __launch_bounds__(512) em_item_kernel(KArgs A, int item_offset) {
     constexpr int T = Shape<MODEL>::T;

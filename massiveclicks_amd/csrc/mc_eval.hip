@@ -7,8 +7,8 @@
 //
 // Three session layouts feed the same per-session arithmetic:
 //   * the caller's arrays, session-major ([n][10] int32 pair indices and
-//     [n][10] click bytes), uploaded per call (mc_evaluate,
-//     mc_serp_probability);
+//     [n][10] click bytes), in pinned chunks of host arrays (mc_evaluate,
+//     mc_serp_probability) or on the device (mc_evaluate_device);
 //   * a held-out set kept resident on the device (mc_set_test_set): sessions
 //     reordered so that the sessions of one query are adjacent (their value
 //     gathers then share cache lines), with the permutation back to the

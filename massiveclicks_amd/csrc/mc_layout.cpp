@@ -72,7 +72,7 @@ void choose_shape(mc_model* m, int64_t n, bool uneven) {
 // entries gets a window of its own as long as two workgroups fit a CU's LDS;
 // one 64-bit atomic to L2 per shown document otherwise bounds its items.  1M
 // UBM sessions on 1,500 queries of up to 1,500 documents: 432 us per
-// iteration with global atomics, 36 us with wide windows.
+// iteration with global atomics, 30 us with wide windows.
 int wide_window(const mc_model* m, int W) {
     if (m->item_window_set || m->reduce_mode != MC_REDUCE_SEGMENTED) return W;
     const size_t budget = 78 * 1024 - window_lds_bytes(m->type, m->reduce_mode, 0);
