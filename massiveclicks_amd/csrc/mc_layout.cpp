@@ -38,14 +38,14 @@ void choose_shape(mc_model* m, int64_t n, bool uneven) {
     // CU; the DBN's two tables and the UBM's examination slots (30 KB) let
     // five, so 512 lanes share a window there, and on sets too small to fill
     // the chip, where more lanes shorten an item.  8M sessions, us per
-    // iteration with 256 / 512 lanes: PBM 69 / 81, CCM 88 / 102, DBN 87 / 83,
-    // UBM 106 / 80; 200,000 sessions: PBM 11.6 / 10.6, CCM 13.1 / 11.6.
+    // iteration with 256 / 512 lanes: PBM 58 / 69, CCM 72 / 83, DBN 80 / 75,
+    // UBM 80 / 74; 200,000 sessions: PBM 10.2 / 9.0, CCM 11.6 / 10.7.
     // The sessions per item grow with the set so that about a thousand items
     // (one or two per resident workgroup) hold the heavy queries: the largest
     // item ends the launch, and each slice of a query adds its flush.  With
-    // 8192 sessions whatever the set, 32,000 PBM sessions took 31 us per
-    // iteration (256: 8), 500,000 DBN sessions 46 (1953: 15), 2M CCM sessions
-    // 72 (1953: 33).
+    // 8192 sessions whatever the set, 32,000 PBM sessions take 19.6 us per
+    // iteration (256: 7.5), 500,000 DBN sessions 26 (1953: 14), 2M CCM
+    // sessions 58 (1953: 27).
     const bool small_window = m->type == MC_PBM || m->type == MC_CCM;
     if (!m->block_set) m->block = small_window && n >= 1000000 ? 256 : 512;
     if (!m->item_sessions_set) {
