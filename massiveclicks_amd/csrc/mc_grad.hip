@@ -840,6 +840,31 @@ void launch_grad_t(mc_model* m, const GArgs& G0, int batch) {
     launch_merge<MODEL, ADAM>(m, Gb);
 }
 
+// The finalisation of batch b - 1 where batch b has no sessions (a query of
+// more than two minibatches' sessions leaves such batches behind it) and so no
+// item launch that carries it: the merge kernel, from version `rd` of the
+// shared state to version `wr`.  It clears all three slots of shared sums:
+// that of b - 1 is read here for the last time, b adds nothing to its own, and
+// the third is the next step's.
+template <int MODEL>
+void launch_carried_step_t(mc_model* m, int b, float* const* rd, float* const* wr, bool wr_main) {
+    GArgs G = make_gargs(m, b - 1);
+    G.shared_off = m->shared_off[(size_t)b - 1];
+    G.shared_cnt = m->shared_cnt[(size_t)b - 1];
+    G.sh_logit = rd[0];
+    G.sh_am = rd[1];
+    G.sh_av = rd[2];
+    G.sh_val = rd[3];
+    G.wr_logit = wr[0];
+    G.wr_am = wr[1];
+    G.wr_av = wr[2];
+    G.wr_val = wr[3];
+    G.wr_main = wr_main;
+    G.sh_acc = m->d_gsh + (size_t)((b - 1) % 3) * kShAccSlot;
+    G.zero_acc = m->d_gsh;
+    launch_merge<MODEL, true>(m, G);
+}
+
 // One Adam step of an epoch replayed from a graph: the step of batch b also
 // finalises the step of batch b - 1 (its split entries and the shared
 // tables), so an epoch is one launch per step plus a closing merge.  The
@@ -880,6 +905,10 @@ void launch_fused_step_t(mc_model* m, int b) {
         }
         const size_t bi = (size_t)b;
         const int64_t nw = m->win_cnt[bi], ng = m->glob_cnt[bi];
+        if (nw + ng == 0) {
+            if (b > 0) launch_carried_step_t<MODEL>(m, b, rd, wr, wr == A4);
+            return;
+        }
         const bool wide = wide_items(m, nw + ng);
         if (nw > 0) {
             if (wide) launch_items<MODEL, true, true, 1024>(m, G, nw, m->win_off[bi], grad_lds_bytes(m));
