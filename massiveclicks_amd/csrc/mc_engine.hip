@@ -685,6 +685,8 @@ void release(mc_model* m) {
     for (void* p : m->allocations) (void)hipFree(p);
     m->allocations.clear();
     m->mem_bytes = 0;
+    // What later calls allocate when they first need it.
+    for (float*& d : m->d_den_user) d = nullptr;
     m->d_test_packed = nullptr;
     m->d_test_pidx = nullptr;
     m->d_test_mask = nullptr;
