@@ -38,23 +38,25 @@ typedef enum {
     MC_ERR_UNSUPPORTED = 6
 } mc_status;
 
-/* Options for mc_model_set_option. */
+/* Options for mc_model_set_option.  MC_AUTO: the library chooses the value
+ * for the training set (the default of the options that take it). */
+enum { MC_AUTO = -1 };
 enum {
     /* 0 = deterministic segmented reduction (default), 1 = float atomics. */
     MC_OPT_REDUCE_MODE = 0,
-    /* Target sessions per workgroup work item (default: chosen for the
-     * training set, 256 to 16384; 8192 in the float-atomic mode). */
+    /* Target sessions per workgroup work item, or MC_AUTO (256 to 16384 by
+     * the training set; 8192 in the float-atomic mode). */
     MC_OPT_ITEM_SESSIONS = 1,
-    /* Per-qd accumulator window per work item, in entries (default 1280, or
-     * up to 2048 for a million sessions and more, with a window of its own
-     * for a query of more entries, as far as LDS goes; when set, such queries
-     * use global atomics). */
+    /* Per-qd accumulator window per work item, in entries, or MC_AUTO (1280,
+     * or up to 2048 for a million sessions and more, with a window of its own
+     * for a query of more entries, as far as LDS goes; with a value, such
+     * queries use global atomics). */
     MC_OPT_ITEM_WINDOW = 2,
     /* 1 = reorder sessions inside each work item by length, then last-click
      * rank, so that wavefronts run uniform chains (default 1). */
     MC_OPT_SORT_BY_LCR = 3,
-    /* Workgroup size of the E/M kernel: 64, 128, 256 or 512 (default: 256 or
-     * 512, chosen for the model and the training set). */
+    /* Workgroup size of the E/M kernel: 64, 128, 256 or 512, or MC_AUTO (256
+     * or 512 by the model and the training set). */
     MC_OPT_BLOCK = 4,
     /* 1 = sessions that are the only session of their query (and show
      * distinct documents) update their entries directly, without a
@@ -283,10 +285,11 @@ mc_status mc_get_session_formats(const mc_model* m, int64_t* n_packed, int64_t* 
 /* Autotuner of the EM work decomposition; no counterpart in the reference
  * (whose launch shape is fixed: BLOCK_SIZE 128, one session per thread).
  * options[MC_N_OPTIONS] holds the starting option values on entry (a
- * candidate itself) and the fastest found on exit.  Each candidate is
- * measured as `iterations` EM iterations replayed from a graph on `device`
- * on this training set (arguments as mc_init_parameters): the reduction mode
- * first, then sessions per work item (512..16384, i.e. sessions per lane),
+ * candidate itself) and the fastest found on exit; the shape that the library
+ * chooses by itself is a candidate too, of which the window stays MC_AUTO.
+ * Each candidate is measured as `iterations` EM iterations replayed from a
+ * graph on `device` on this training set (arguments as mc_init_parameters):
+ * the reduction mode first, then sessions per work item (512..16384, i.e. sessions per lane),
  * the LDS window, the lanes per work item (256 or 512) and the session
  * format (MC_OPT_PACKED).  *best_ms_per_iter and *n_trials report the
  * winner's time and the number of candidates measured. */

@@ -211,7 +211,7 @@ int main(int argc, char** argv) {
 
         // ---- EM (parallel_em.cu:349-609) ------------------------------------
         const auto t_em = std::chrono::steady_clock::now();
-        int64_t opts[MC_N_OPTIONS] = {config.reduce_mode, 8192, 1280, 1, 256, 0, 1, 1, 1, 1, 1};
+        int64_t opts[MC_N_OPTIONS] = {config.reduce_mode, MC_AUTO, MC_AUTO, 1, MC_AUTO, 0, 1, 1, 1, 1, 1};
         if (config.autotune) {
             const mclicks::Sessions tr = ds.train();
             double ms = 0.0;
@@ -219,16 +219,14 @@ int main(int argc, char** argv) {
             mclicks::check(mc_autotune(config.model_type, 0, tr.size(), tr.query.data(), tr.pidx.data(),
                                        tr.clicks.data(), nullptr, ds.n_qd(), 5, opts, &ms, &trials));
             std::cout << "\nAutotune (" << trials << " candidates): reduce-mode " << opts[MC_OPT_REDUCE_MODE]
-                      << ", item-sessions " << opts[MC_OPT_ITEM_SESSIONS] << ", window " << opts[MC_OPT_ITEM_WINDOW]
-                      << ", block " << opts[MC_OPT_BLOCK] << ": " << ms
-                      << " ms/iteration" << std::endl;
+                      << ", item-sessions " << opts[MC_OPT_ITEM_SESSIONS] << ", window "
+                      << (opts[MC_OPT_ITEM_WINDOW] == MC_AUTO ? std::string("automatic")
+                                                              : std::to_string(opts[MC_OPT_ITEM_WINDOW]))
+                      << ", block " << opts[MC_OPT_BLOCK] << ": " << ms << " ms/iteration" << std::endl;
         }
         if (config.fit == "adam") opts[MC_OPT_BATCHES] = std::max(1, config.batches);
         mclicks::ClickModel cm(config.model_type, 0);
-        // Options that nothing has chosen keep the library's defaults, which
-        // it picks for the training set.
-        for (int o = 0; o < MC_N_OPTIONS; o++)
-            if (config.autotune || o == MC_OPT_REDUCE_MODE || o == MC_OPT_BATCHES) cm.set_option(o, opts[o]);
+        for (int o = 0; o < MC_N_OPTIONS; o++) cm.set_option(o, opts[o]);
         const auto t_h2d = std::chrono::steady_clock::now();
         cm.init_parameters(ds);
         const double h2d_s = seconds_since(t_h2d);

@@ -1031,14 +1031,15 @@ mc_status mc_model_set_option(mc_model* m, int option, int64_t value) {
             m->reduce_mode = (int)value;
             break;
         case MC_OPT_ITEM_SESSIONS:
-            MC_REQUIRE(value >= 64 && value <= (1 << 20), "item sessions out of range [64, 2^20]");
+            MC_REQUIRE(value == MC_AUTO || (value >= 64 && value <= (1 << 20)),
+                       "item sessions out of range [64, 2^20]");
             m->item_sessions = (int)value;
-            m->item_sessions_set = true;
+            m->item_sessions_set = value != MC_AUTO;
             break;
         case MC_OPT_ITEM_WINDOW:
-            MC_REQUIRE(value >= 0 && value <= 16384, "item window out of range [0, 16384]");
+            MC_REQUIRE(value == MC_AUTO || (value >= 0 && value <= 16384), "item window out of range [0, 16384]");
             m->item_window = (int)value;
-            m->item_window_set = true;
+            m->item_window_set = value != MC_AUTO;
             break;
         case MC_OPT_SORT_BY_LCR:
             m->sort_by_lcr = value != 0;
@@ -1062,9 +1063,10 @@ mc_status mc_model_set_option(mc_model* m, int option, int64_t value) {
             m->n_batches = (int)value;
             break;
         case MC_OPT_BLOCK:
-            MC_REQUIRE(value == 64 || value == 128 || value == 256 || value == 512, "block must be 64/128/256/512");
+            MC_REQUIRE(value == MC_AUTO || value == 64 || value == 128 || value == 256 || value == 512,
+                       "block must be 64/128/256/512");
             m->block = (int)value;
-            m->block_set = true;
+            m->block_set = value != MC_AUTO;
             break;
         default:
             set_error("unknown option");

@@ -23,6 +23,7 @@ MAX_SERP = 10
 (OPT_REDUCE_MODE, OPT_ITEM_SESSIONS, OPT_ITEM_WINDOW, OPT_SORT_BY_LCR, OPT_BLOCK, OPT_DIRECT, OPT_PERSISTENT,
  OPT_BATCHES, OPT_PACKED, OPT_SKIP_CONSTANT, OPT_FUSED_MERGE) = range(11)
 REDUCE_SEGMENTED, REDUCE_ATOMIC = 0, 1
+AUTO = -1   # item_sessions, item_window, block: chosen for the training set
 
 
 @dataclass
@@ -371,8 +372,12 @@ class ClickModel:
 
 OPTION_NAMES = ("reduce_mode", "item_sessions", "item_window", "sort_by_lcr", "block", "direct", "persistent",
                 "batches", "packed", "skip_constant", "fused_merge")
-DEFAULT_OPTIONS = {"reduce_mode": REDUCE_SEGMENTED, "item_sessions": 8192, "item_window": 1280, "sort_by_lcr": 1,
-                   "block": 256, "direct": 0, "persistent": 1, "batches": 1, "packed": 1, "skip_constant": 1, "fused_merge": 1}
+DEFAULT_OPTIONS = {"reduce_mode": REDUCE_SEGMENTED, "item_sessions": AUTO, "item_window": AUTO, "sort_by_lcr": 1,
+                   "block": AUTO, "direct": 0, "persistent": 1, "batches": 1, "packed": 1, "skip_constant": 1,
+                   "fused_merge": 1}
+# Part of the cache keys of autotune: a shape found with other kernels, or
+# among other candidates, is not the fastest one any more.
+TUNE_VERSION = 2
 
 
 def autotune(model_type: int, train: SessionSet, n_qd: int, device: int = 0, iterations: int = 5,
@@ -380,10 +385,11 @@ def autotune(model_type: int, train: SessionSet, n_qd: int, device: int = 0, ite
     """Fastest EM options for this model and training set (mc_autotune).
     Returns (options, info): options are keyword arguments of ClickModel,
     info = {ms_per_iter, trials, cached}.  With `cache` (a JSON file) results
-    are stored per (model, sessions, n_qd, uneven lengths) and reused."""
+    are stored per (model, sessions, n_qd, uneven lengths, TUNE_VERSION) and
+    reused."""
     import json
     import os
-    key = f"{MODEL_NAMES[model_type]}:{len(train)}:{n_qd}:{int(train.length is not None)}"
+    key = f"{MODEL_NAMES[model_type]}:{len(train)}:{n_qd}:{int(train.length is not None)}:v{TUNE_VERSION}"
     if cache and os.path.exists(cache):
         with open(cache) as f:
             known = json.load(f)
