@@ -783,30 +783,50 @@ GArgs make_gargs(mc_model* m, int batch) {
     return G;
 }
 
-// Accumulators and staged values of the widest window, the UBM's slots.
+// Accumulators and staged values of the widest window, the UBM's slots.  One
+// launch holds the windows of every width: a query wider than the item window
+// takes LDS from the others' workgroups, but a launch of its own costs more.
+// 480,000 sessions and one such query, us per epoch with one launch / two: PBM
+// 30 / 38, DBN 42 / 49; 3M sessions: PBM 87 / 95, DBN 120 / 123, UBM 77 / 91.
 size_t grad_lds_bytes(const mc_model* m) {
     return window_lds_bytes(m->type, MC_REDUCE_SEGMENTED, std::max(m->max_width, m->wide_width));
 }
 
-// 1024 lanes per item where a launch has few items (a small minibatch: one
-// workgroup per CU then), else 512, which keep 24 to 32 wavefronts on a CU.
-// Adam epochs, us with 1024 / 512 lanes: 700,000 DBN sessions in 729 items
-// 46.5 / 35.5; 1M in three minibatches of 200 items 94 / 119; 256 lanes took
-// 20 more of 126 us on the 1,360 items of the rarest queries.  Items of more
-// than 4096 sessions stay with 1024 lanes up to four per CU (a gradient of 1M
-// sessions in 605 items of up to 8192: 53 / 63 us).
-bool wide_items(const mc_model* m, int64_t n_items) {
-    return 2 * n_items < 3 * (int64_t)m->n_cu || (n_items < 4 * (int64_t)m->n_cu && m->max_item_sessions > 4096);
+// Lanes per item of list b.  A CU holds one workgroup of 1024 lanes (79-128
+// VGPRs), so 1024 lanes pay where one round of items runs and its sessions
+// take more than one pass of 512: equal DBN items of 1,000 entries, us per
+// epoch with 512 / 1024 lanes: 250 items of 300 sessions 20 / 20, of 1,500
+// 25 / 23, of 6,000 46 / 38; 270 items 22 / 27, 28 / 31, 54 / 58.  Up to one
+// and a half rounds they also pay where a large item would end the launch (3M
+// UBM sessions, Zipf(1.4), four minibatches of about 200 items of up to 5,853
+// sessions: 118 / 92).  Many items are better off with 256 lanes, which leave
+// fewer idle in an item's last pass, as long as eight such workgroups' windows
+// fit a CU's LDS (PBM and CCM): 1,500 PBM items, with 256 / 512 lanes, of 300
+// sessions 33 / 39, of 1,500 44 / 49; 2M Zipf(1.1) sessions CCM 51 / 56, DBN
+// (38 KB windows) 63 / 60; 600 CCM items of 1,500 sessions 35 / 34.
+int item_lanes(const mc_model* m, size_t b) {
+    const int64_t n_items = m->win_cnt[b] + m->glob_cnt[b], largest = m->largest_item[b];
+    if (n_items <= (int64_t)m->n_cu && largest > 512) return 1024;
+    if (2 * n_items <= 3 * (int64_t)m->n_cu && largest > 2048) return 1024;
+    if (n_items >= 4 * (int64_t)m->n_cu && grad_lds_bytes(m) <= 20000) return 256;
+    return 512;
 }
 
 template <int MODEL, bool WIN, bool ADAM, int NT>
-void launch_items(mc_model* m, const GArgs& G, int64_t count, int64_t off, size_t lds) {
+void launch_items_of(mc_model* m, const GArgs& G, int64_t count, int64_t off, size_t lds) {
     if (m->varlen)
         hipLaunchKernelGGL((grad_item_kernel<MODEL, true, WIN, ADAM, NT>), dim3((unsigned)count), dim3(NT), lds,
                            m->stream, G, off);
     else
         hipLaunchKernelGGL((grad_item_kernel<MODEL, false, WIN, ADAM, NT>), dim3((unsigned)count), dim3(NT), lds,
                            m->stream, G, off);
+}
+
+template <int MODEL, bool WIN, bool ADAM>
+void launch_items(mc_model* m, const GArgs& G, int lanes, int64_t count, int64_t off, size_t lds) {
+    if (lanes == 1024) launch_items_of<MODEL, WIN, ADAM, 1024>(m, G, count, off, lds);
+    else if (lanes == 512) launch_items_of<MODEL, WIN, ADAM, 512>(m, G, count, off, lds);
+    else launch_items_of<MODEL, WIN, ADAM, 256>(m, G, count, off, lds);
 }
 
 // The merge in one block while that takes one pass over its split entries,
@@ -827,15 +847,9 @@ void launch_grad_t(mc_model* m, const GArgs& G0, int batch) {
     Gb.shared_off = m->shared_off[b];
     Gb.shared_cnt = m->shared_cnt[b];
     const GArgs& G = Gb;
-    const bool wide = wide_items(m, nw + ng);
-    if (nw > 0) {
-        if (wide) launch_items<MODEL, true, ADAM, 1024>(m, G, nw, m->win_off[b], grad_lds_bytes(m));
-        else launch_items<MODEL, true, ADAM, 512>(m, G, nw, m->win_off[b], grad_lds_bytes(m));
-    }
-    if (ng > 0) {
-        if (wide) launch_items<MODEL, false, ADAM, 1024>(m, G, ng, m->glob_off[b], 0);
-        else launch_items<MODEL, false, ADAM, 512>(m, G, ng, m->glob_off[b], 0);
-    }
+    const int lanes = item_lanes(m, b);
+    if (nw > 0) launch_items<MODEL, true, ADAM>(m, G, lanes, nw, m->win_off[b], grad_lds_bytes(m));
+    if (ng > 0) launch_items<MODEL, false, ADAM>(m, G, lanes, ng, m->glob_off[b], 0);
     Gb.end_epoch = ADAM && batch == m->n_batches - 1;
     launch_merge<MODEL, ADAM>(m, Gb);
 }
@@ -909,11 +923,8 @@ void launch_fused_step_t(mc_model* m, int b) {
             if (b > 0) launch_carried_step_t<MODEL>(m, b, rd, wr, wr == A4);
             return;
         }
-        const bool wide = wide_items(m, nw + ng);
-        if (nw > 0) {
-            if (wide) launch_items<MODEL, true, true, 1024>(m, G, nw, m->win_off[bi], grad_lds_bytes(m));
-            else launch_items<MODEL, true, true, 512>(m, G, nw, m->win_off[bi], grad_lds_bytes(m));
-        }
+        const int lanes = item_lanes(m, bi);
+        if (nw > 0) launch_items<MODEL, true, true>(m, G, lanes, nw, m->win_off[bi], grad_lds_bytes(m));
         if (ng > 0) {
             // A second launch of the same step: the finalisation is done and
             // the shared values are in the written version.
@@ -921,8 +932,7 @@ void launch_fused_step_t(mc_model* m, int b) {
                 G.prev_batch = -1;
                 G.sh_val = G.wr_val;
             }
-            if (wide) launch_items<MODEL, false, true, 1024>(m, G, ng, m->glob_off[bi], 0);
-            else launch_items<MODEL, false, true, 512>(m, G, ng, m->glob_off[bi], 0);
+            launch_items<MODEL, false, true>(m, G, lanes, ng, m->glob_off[bi], 0);
         }
         return;
     }

@@ -59,12 +59,16 @@ void choose_shape(mc_model* m, int64_t n, bool uneven) {
     // many: UBM 8M 81.5 / 71.4, 1M 19.8 / 18.3; DBN 8M 76.7 / 74.0, 1M 20.4 /
     // 18.5, 2M 28.7 / 28.9; CCM 8M 71.0 / 70.5, 2M 28.2 / 26.9.  Small sets
     // are better off with more items (500,000 DBN 14.4 / 14.1, 312,000 UBM
-    // 10.8 / 11.0), the PBM gains nothing (8M 56.6 / 56.3, 2M 23.2 / 23.6).
+    // 10.8 / 11.0), the PBM gains nothing (8M 56.6 / 56.3, 2M 23.2 / 23.6);
+    // so are small minibatches, whose steps have few items to spread over the
+    // chip (1M DBN sessions in eight, us per Adam epoch with 1280 / 1600: 127 /
+    // 134; 2M in four, 131 / 114).
     if (!m->item_window_set) {
         m->item_window = 1280;
-        if (n >= 1000000 && m->block == 512 && m->type == MC_UBM) m->item_window = 2048;
-        if (n >= 1000000 && m->block == 512 && m->type == MC_DBN) m->item_window = 1600;
-        if (n >= 1000000 && m->block == 256 && m->type == MC_CCM) m->item_window = 1504;
+        const bool large = n >= 1000000 && n / m->n_batches >= 200000;
+        if (large && m->block == 512 && m->type == MC_UBM) m->item_window = 2048;
+        if (large && m->block == 512 && m->type == MC_DBN) m->item_window = 1600;
+        if (large && m->block == 256 && m->type == MC_CCM) m->item_window = 1504;
     }
 }
 
@@ -457,7 +461,12 @@ mc_status plan_layout(mc_model* m, int64_t n, const int32_t* query, const int32_
         m->glob_off.assign((size_t)B + 1, 0);
         m->glob_cnt.assign((size_t)B + 1, 0);
         m->batch_sessions.assign((size_t)B, 0);
-        for (const Item& it : items) m->batch_sessions[(size_t)it.pad] += it.s1 - it.s0;
+        m->largest_item.assign((size_t)B + 1, 0);
+        for (const Item& it : items) {
+            m->batch_sessions[(size_t)it.pad] += it.s1 - it.s0;
+            for (int b : {(int)it.pad, B})
+                m->largest_item[(size_t)b] = std::max<int64_t>(m->largest_item[(size_t)b], it.s1 - it.s0);
+        }
         const int g0 = m->n_win_items, g1 = m->n_win_items + m->n_glob_items;
         for (int b = 0; b <= B; b++) {
             m->win_off[(size_t)b] = (int64_t)lists.size();
