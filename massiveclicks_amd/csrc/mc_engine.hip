@@ -605,13 +605,6 @@ __global__ void __launch_bounds__(256) em_merge_kernel(KArgs A) {
     }
 }
 
-// Denominators of per-qd table t after an M-step: entries [first, first + n).
-template <int MODEL>
-__global__ void __launch_bounds__(256) den_kernel(const int2* counts, int t, float* out, int64_t first, int64_t n) {
-    const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < n) out[i] = base_den<MODEL>(t, counts[first + i]).y;
-}
-
 // Copies n 4-byte words to pinned host memory, 16 bytes a lane.
 __global__ void __launch_bounds__(256) copy_out_kernel(const uint32_t* src, uint32_t* out, int64_t n) {
     const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
@@ -721,35 +714,46 @@ mc_status stage_reserve(mc_model* m, size_t bytes) {
 
 namespace {
 // Host array of n bytes from chunks that produce(dst, offset, bytes) enqueues
-// into pinned memory.  The copies out of the pinned chunks are spread over a
-// few threads: the destination is usually fresh memory, whose page faults
-// cost one thread more than the link does.  A 27 MB table's numerators and
-// denominators into new numpy arrays: 6.9 ms by the runtime's pageable copy
-// (17 GB/s) and a loop over the counts on the host, 3.9 so with two threads,
-// 2.7 with four or eight.
+// into pinned memory; beside(offset, bytes) is the host's own work for the
+// same range, done while the chunk is on its way.  The copies out of the
+// pinned chunks are spread over a few threads: the destination is usually
+// fresh memory, whose page faults cost one thread more than the link does.
+// Numerators and denominators of a table into new numpy arrays, us by the
+// runtime's pageable copy and a loop over the counts / so: 2,000 entries 21 /
+// 18, 90,000 38 / 35, 250,000 83 / 68, 4M 1,900 / 490.  (Denominators by a
+// kernel and a second pass: 31, 56, 101 and 840.)
 constexpr size_t kStageChunk = (size_t)1 << 20;
 constexpr size_t kStageSmallChunk = (size_t)256 << 10;
 constexpr size_t kStageThreadsFrom = (size_t)8 << 20;   // below, starting threads costs more than they save
-// About four chunks of a small array, so that copies overlap.
+// One chunk up to 1 MB: an event costs as much as the overlap saves (130,000
+// entries 42 us in one chunk, 46 in two; 250,000 68, 79 in four).  About four
+// chunks of a somewhat larger array, so that copies overlap.
 size_t stage_chunk(size_t n) {
-    return std::min(n, std::min(kStageChunk, std::max(kStageSmallChunk, (n / 4 + 255) / 256 * 256)));
+    if (n <= kStageChunk) return n;
+    return std::min(kStageChunk, std::max(kStageSmallChunk, (n / 4 + 255) / 256 * 256));
 }
-template <class Produce>
-mc_status staged_out(mc_model* m, char* dst, size_t n, Produce produce) {
+// Bytes of each of the kStages slots, which lie side by side: a single chunk
+// takes as many of them as it needs.
+size_t stage_slot(size_t n) { return n <= kStageChunk ? (n + kStages - 1) / kStages : stage_chunk(n); }
+template <class Produce, class Beside>
+mc_status staged_out(mc_model* m, char* dst, size_t n, Produce produce, Beside beside) {
     if (n == 0) return MC_OK;
     const size_t chunk = stage_chunk(n);
-    MC_TRY(stage_reserve(m, chunk));
+    MC_TRY(stage_reserve(m, stage_slot(n)));
     const size_t chunks = (n + chunk - 1) / chunk;
     auto size_of = [&](size_t k) { return std::min(chunk, n - k * chunk); };
     auto copy_here = [&]() -> mc_status {   // by this thread alone
         for (size_t k = 0; k < chunks + kStages - 1; k++) {
             if (k < chunks) {
                 MC_TRY(produce(m->stage[k % kStages], k * chunk, size_of(k)));
-                if (chunks > 1) MC_HIP(hipEventRecord(m->stage_ev[k % kStages], m->stream));
+                if (k + 1 < chunks) MC_HIP(hipEventRecord(m->stage_ev[k % kStages], m->stream));
+                beside(k * chunk, size_of(k));
             }
             if (k + 1 < kStages) continue;
             const size_t j = k + 1 - kStages;
-            if (chunks > 1) MC_HIP(hipEventSynchronize(m->stage_ev[j % kStages]));
+            // The stream's end instead of the last event: the next call's
+            // first launch otherwise takes 20 us longer.
+            if (j + 1 < chunks) MC_HIP(hipEventSynchronize(m->stage_ev[j % kStages]));
             else MC_HIP(hipStreamSynchronize(m->stream));
             std::memcpy(dst + j * chunk, m->stage[j % kStages], size_of(j));
         }
@@ -763,6 +767,7 @@ mc_status staged_out(mc_model* m, char* dst, size_t n, Produce produce) {
     // k % kStages, whose use number is k / kStages.
     auto work = [&](size_t w, size_t W) {
         for (size_t k = w; k < chunks; k += W) {
+            beside(k * chunk, size_of(k));
             while (issued.load(std::memory_order_acquire) <= k) {
                 if (error.load() != (int)hipSuccess) return;
                 std::this_thread::yield();
@@ -804,21 +809,33 @@ mc_status staged_out(mc_model* m, char* dst, size_t n, Produce produce) {
     return st;
 }
 
-template <int MODEL>
-void launch_den(mc_model* m, int t, float* out, int64_t first, int64_t n) {
-    hipLaunchKernelGGL(den_kernel<MODEL>, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, m->stream, m->d_counts, t, out,
-                       first, n);
+// Enqueues a copy of a chunk.
+mc_status copy_out(mc_model* m, const void* src, char* to, size_t at, size_t bytes) {
+    const int64_t words = (int64_t)(bytes / 4);
+    hipLaunchKernelGGL(copy_out_kernel, dim3((unsigned)((words + 1023) / 1024)), dim3(256), 0, m->stream,
+                       (const uint32_t*)((const char*)src + at), (uint32_t*)to, words);
+    MC_HIP(hipGetLastError());
+    return MC_OK;
+}
+
+// Denominators of per-qd table t after an M-step, as base_den in the kernels:
+// entries [first, first + n).
+void constant_den(const mc_model* m, int t, float* out, size_t first, size_t n) {
+    const int2* c = m->h_counts.data() + first;
+    out += first;
+    if (m->type == MC_CCM)
+        for (size_t i = 0; i < n; i++) out[i] = 2.f + (float)c[i].x + (float)c[i].y;
+    else if (m->type == MC_DBN && t == 1)
+        for (size_t i = 0; i < n; i++) out[i] = 2.f + 2.f * (float)c[i].x - (float)c[i].y;
+    else
+        for (size_t i = 0; i < n; i++) out[i] = 2.f + (float)c[i].x;
 }
 }  // namespace
 
 mc_status download(mc_model* m, void* dst, const void* src, size_t n) {
-    return staged_out(m, (char*)dst, n, [&](char* to, size_t at, size_t bytes) -> mc_status {
-        const int64_t words = (int64_t)(bytes / 4);
-        hipLaunchKernelGGL(copy_out_kernel, dim3((unsigned)((words + 1023) / 1024)), dim3(256), 0, m->stream,
-                           (const uint32_t*)((const char*)src + at), (uint32_t*)to, words);
-        MC_HIP(hipGetLastError());
-        return MC_OK;
-    });
+    return staged_out(
+        m, (char*)dst, n, [&](char* to, size_t at, size_t bytes) { return copy_out(m, src, to, at, bytes); },
+        [](size_t, size_t) {});
 }
 
 mc_status fill(mc_model* m, float* p, float v, int64_t n) {
@@ -1215,8 +1232,9 @@ mc_status mc_init_parameters(mc_model* m, int64_t n, const int32_t* query, const
     }
     m->den_state[T] = 0;
     // For the tables' readback and evaluations of a few thousand host rows.
-    MC_TRY(stage_reserve(m, std::max(stage_chunk((size_t)n_qd * 4), (size_t)64 << 10)));
+    MC_TRY(stage_reserve(m, std::max(stage_slot((size_t)n_qd * 4), (size_t)64 << 10)));
     MC_HIP(hipStreamSynchronize(m->stream));
+    m->h_counts = std::move(h.counts);
     m->cur = 0;
     m->estep_pending = false;
     m->initialized = true;
@@ -1373,26 +1391,24 @@ mc_status mc_get_parameters(mc_model* m, int t, float* num, float* den) {
         if (den) std::fill(den, den + n, 1.f);
         return MC_OK;
     }
-    if (num) MC_TRY(download(m, num, shared ? m->d_sh_num[m->cur] : m->d_num[m->cur][t], n * 4));
-    if (!den) return MC_OK;
-    if (shared) return download(m, den, m->d_sh_den[m->cur], n * 4);
-    if (m->den_state[t] == 1) return download(m, den, m->d_den_user[t], n * 4);
-    if (m->den_state[t] == 0) {
-        std::fill(den, den + n, 2.f);
-        return MC_OK;
-    }
-    // The M-step's constants, from the counts straight into pinned memory.
-    return staged_out(m, (char*)den, (size_t)n * 4, [&](char* to, size_t at, size_t bytes) -> mc_status {
-        float* out = (float*)to;
-        const int64_t first = (int64_t)(at / 4), k = (int64_t)(bytes / 4);
-        switch (m->type) {
-            case MC_CCM: launch_den<kCCM>(m, t, out, first, k); break;
-            case MC_DBN: launch_den<kDBN>(m, t, out, first, k); break;
-            default: launch_den<kPBM>(m, t, out, first, k); break;
-        }
-        MC_HIP(hipGetLastError());
-        return MC_OK;
-    });
+    // The host fills in denominators that it knows (the prior's, or the
+    // M-step's constants) while the numerators are on their way.
+    const float* src = shared ? m->d_sh_num[m->cur] : m->d_num[m->cur][t];
+    auto host_den = [&](size_t at, size_t bytes) {
+        const size_t first = at / 4, k = bytes / 4;
+        if (!den || shared || m->den_state[t] == 1) return;
+        if (m->den_state[t] == 0) std::fill(den + first, den + first + k, 2.f);
+        else constant_den(m, t, den, first, k);
+    };
+    if (num)
+        MC_TRY(staged_out(
+            m, (char*)num, (size_t)n * 4,
+            [&](char* to, size_t at, size_t bytes) { return copy_out(m, src, to, at, bytes); }, host_den));
+    else
+        host_den(0, (size_t)n * 4);
+    if (den && shared) return download(m, den, m->d_sh_den[m->cur], n * 4);
+    if (den && m->den_state[t] == 1) return download(m, den, m->d_den_user[t], n * 4);
+    return MC_OK;
 }
 
 mc_status mc_set_parameters(mc_model* m, int t, const float* num, const float* den) {
