@@ -204,7 +204,8 @@ mc_status mc_reset_parameters(mc_model* m);
  * pair, valued 1/2), clicks[n*10], len[n] (NULL = 10).  Outputs: logp/full
  * (n*10, nullable), llh[n] per-session mean log-probability (nullable),
  * *llh_sum = sum of llh, ppl_log2_sum[10] = per-rank sums of log2(full)
- * (FP32 partials per device lane over its few sessions, FP64 beyond),
+ * (FP64 sums of FP32 terms; of the resident held-out set, FP32 partials per
+ * device lane over its few sessions, FP64 beyond),
  * rank_count[10] = sessions contributing to each rank.  Without per-session
  * outputs a session's llh is formed from log2 and scaled by ln 2 (within
  * 1e-8 relative of the natural-log sum).  LL = llh_sum / n;

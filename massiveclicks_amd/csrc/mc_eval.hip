@@ -24,6 +24,7 @@
 #include <cstring>
 #include <mutex>
 #include <string>
+#include <type_traits>
 #include <vector>
 
 #include "mclicks.h"
@@ -319,12 +320,17 @@ __global__ void __launch_bounds__(256) eval_kernel(EvalArgs E) {
     __shared__ WaveRows rows[major ? 4 : 1];
     const int tid = threadIdx.x, lane = tid & 63;
     WaveRows& wr = rows[major ? tid >> 6 : 0];
-    // Per-lane FP32 partials of the lane's sessions (a lane takes every
-    // (blocks x 256)-th session, about four of 2M test sessions), FP64 from
-    // the wavefront sums on.
-    float v[11];
+    // Sums of the lane's sessions.  Resident: FP32 partials (a lane takes every
+    // (blocks x 256)-th session, about four of 2M test sessions), FP64 from the
+    // wavefront sums on.  Session-major, where half as many blocks take twice
+    // as many sessions a lane: FP64 throughout (llh_sum of 4M DBN sessions off
+    // by 3e-9 with FP32 partials, by 2e-9 with twice the blocks; 1M sessions
+    // with outputs, us with FP32 / FP64: PBM 40.4 / 40.4, UBM 49.2 / 48.8, CCM
+    // 39.6 / 39.7, DBN 55.9 / 56.1; CCM sums alone 29.7 / 30.4).
+    using Sum = typename std::conditional<major, double, float>::type;
+    Sum v[11];
 #pragma unroll
-    for (int k = 0; k < 11; k++) v[k] = 0.f;
+    for (int k = 0; k < 11; k++) v[k] = 0;
     int cnt[kL];
 #pragma unroll
     for (int r = 0; r < kL; r++) cnt[r] = 0;
@@ -391,13 +397,13 @@ __global__ void __launch_bounds__(256) eval_kernel(EvalArgs E) {
             if (r < L) acc = acc + lp[r];
         if (!OUT) acc *= 0.693147180559945309f;   // log2 sum to natural log
         const float s = acc / L;                 // evaluation.cpp:36
-        if (real) v[0] += s;
+        if (real) v[0] += (Sum)s;
         const int64_t o = (OUT && !major && E.perm && real) ? (int64_t)E.perm[i] : i;
         if (OUT && E.llh && real) E.llh[o] = s;
 #pragma unroll
         for (int r = 0; r < kL; r++) {
             cnt[r] += (int)__popcll(__ballot(r < L && real));
-            if (r < L && real) v[1 + r] += log2f(fp[r]);   // evaluation.cpp:62
+            if (r < L && real) v[1 + r] += (Sum)log2f(fp[r]);   // evaluation.cpp:62
             if (OUT && !major && E.logp && real) E.logp[o * kL + r] = r < L ? lp[r] : 0.f;
             if (OUT && !major && E.full && real) E.full[o * kL + r] = r < L ? fp[r] : 0.f;
         }
