@@ -821,14 +821,22 @@ mc_status copy_out(mc_model* m, const void* src, char* to, size_t at, size_t byt
 // Denominators of per-qd table t after an M-step, as base_den in the kernels:
 // entries [first, first + n).
 void constant_den(const mc_model* m, int t, float* out, size_t first, size_t n) {
-    const int2* c = m->h_counts.data() + first;
-    out += first;
-    if (m->type == MC_CCM)
-        for (size_t i = 0; i < n; i++) out[i] = 2.f + (float)c[i].x + (float)c[i].y;
-    else if (m->type == MC_DBN && t == 1)
-        for (size_t i = 0; i < n; i++) out[i] = 2.f + 2.f * (float)c[i].x - (float)c[i].y;
+    // All from the packed counts, then those that do not fit there.
+    const int kind = m->type == MC_CCM ? 2 : m->type == MC_DBN && t == 1 ? 1 : 0;
+    auto den = [kind](int o, int c) {
+        return kind == 2 ? 2.f + (float)o + (float)c : kind == 1 ? 2.f + 2.f * (float)o - (float)c : 2.f + (float)o;
+    };
+    const uint16_t* c = m->h_counts16.data();
+    if (kind == 2)
+        for (size_t i = first; i < first + n; i++) out[i] = 2.f + (float)(c[i] & 0xff) + (float)(c[i] >> 8);
+    else if (kind == 1)
+        for (size_t i = first; i < first + n; i++) out[i] = 2.f + 2.f * (float)(c[i] & 0xff) - (float)(c[i] >> 8);
     else
-        for (size_t i = 0; i < n; i++) out[i] = 2.f + (float)c[i].x;
+        for (size_t i = first; i < first + n; i++) out[i] = 2.f + (float)(c[i] & 0xff);
+    auto big = std::lower_bound(m->h_big_counts.begin(), m->h_big_counts.end(), first,
+                                [](const mc_model::BigCount& b, size_t p) { return (size_t)b.entry < p; });
+    for (; big != m->h_big_counts.end() && (size_t)big->entry < first + n; ++big)
+        out[big->entry] = den(big->counts.x, big->counts.y);
 }
 }  // namespace
 
@@ -1210,9 +1218,12 @@ mc_status mc_init_parameters(mc_model* m, int64_t n, const int32_t* query, const
         MC_HIP(hipMemcpyAsync(m->d_lists, lists.data(), lists.size() * 4, hipMemcpyHostToDevice, m->stream));
     MC_HIP(hipMemcpyAsync(m->d_counts, counts.data(), counts.size() * 8, hipMemcpyHostToDevice, m->stream));
     std::vector<uint16_t> counts16((size_t)n_qd);
-    for (int64_t p = 0; p < n_qd; p++)
-        counts16[(size_t)p] = counts[(size_t)p].x < 255 ? (uint16_t)(counts[(size_t)p].x | (counts[(size_t)p].y << 8))
-                                                      : (uint16_t)kCountsEscape;
+    m->h_big_counts.clear();
+    for (int64_t p = 0; p < n_qd; p++) {
+        const int2 c = counts[(size_t)p];
+        counts16[(size_t)p] = c.x < 255 ? (uint16_t)(c.x | (c.y << 8)) : (uint16_t)kCountsEscape;
+        if (c.x >= 255) m->h_big_counts.push_back({(int32_t)p, c});
+    }
     MC_HIP(hipMemcpyAsync(m->d_counts16, counts16.data(), counts16.size() * 2, hipMemcpyHostToDevice, m->stream));
     MC_HIP(hipMemcpyAsync(m->d_sh_base, sh_base.data(), sh_base.size() * 8, hipMemcpyHostToDevice, m->stream));
     MC_HIP(hipMemcpyAsync(m->d_sh_acc_map, sh_map.data(), sh_map.size() * 4, hipMemcpyHostToDevice, m->stream));
@@ -1234,7 +1245,7 @@ mc_status mc_init_parameters(mc_model* m, int64_t n, const int32_t* query, const
     // For the tables' readback and evaluations of a few thousand host rows.
     MC_TRY(stage_reserve(m, std::max(stage_slot((size_t)n_qd * 4), (size_t)64 << 10)));
     MC_HIP(hipStreamSynchronize(m->stream));
-    m->h_counts = std::move(h.counts);
+    m->h_counts16 = std::move(counts16);
     m->cur = 0;
     m->estep_pending = false;
     m->initialized = true;

@@ -79,7 +79,14 @@ struct mc_model {
     float* d_num[2][2] = {{nullptr, nullptr}, {nullptr, nullptr}};
     int2* d_counts = nullptr;
     uint16_t* d_counts16 = nullptr;  // packed counts read by the window flushes
-    std::vector<int2> h_counts;      // host copy of d_counts, for the denominators read back
+    // Host copies for the denominators read back: d_counts16, and the counts
+    // that do not fit there, in ascending order.
+    std::vector<uint16_t> h_counts16;
+    struct BigCount {
+        int32_t entry;
+        int2 counts;
+    };
+    std::vector<BigCount> h_big_counts;
     unsigned long long* d_gacc[2] = {nullptr, nullptr};
     float* d_den_user[2] = {nullptr, nullptr};
     int den_state[3] = {0, 0, 0};  // per table: 0 prior (2), 1 user-set, 2 M-step constant, 3 value only
