@@ -797,17 +797,19 @@ size_t grad_lds_bytes(const mc_model* m) {
 // take more than one pass of 512: equal DBN items of 1,000 entries, us per
 // epoch with 512 / 1024 lanes: 250 items of 300 sessions 20 / 20, of 1,500
 // 25 / 23, of 6,000 46 / 38; 270 items 22 / 27, 28 / 31, 54 / 58.  Up to one
-// and a half rounds they also pay where a large item would end the launch (3M
-// UBM sessions, Zipf(1.4), four minibatches of about 200 items of up to 5,853
-// sessions: 118 / 92).  Many items are better off with 256 lanes, which leave
+// and a half rounds they also pay where an item larger than the others would
+// end the launch (3M UBM sessions, Zipf(1.4), four minibatches of about 200
+// items of up to 5,853 sessions: 118 / 92; 258 equal CCM items of 3,400
+// sessions 34 / 39).  Many items are better off with 256 lanes, which leave
 // fewer idle in an item's last pass, as long as eight such workgroups' windows
 // fit a CU's LDS (PBM and CCM): 1,500 PBM items, with 256 / 512 lanes, of 300
 // sessions 33 / 39, of 1,500 44 / 49; 2M Zipf(1.1) sessions CCM 51 / 56, DBN
 // (38 KB windows) 63 / 60; 600 CCM items of 1,500 sessions 35 / 34.
 int item_lanes(const mc_model* m, size_t b) {
     const int64_t n_items = m->win_cnt[b] + m->glob_cnt[b], largest = m->largest_item[b];
+    const int64_t sessions = b < m->batch_sessions.size() ? m->batch_sessions[b] : m->N;
     if (n_items <= (int64_t)m->n_cu && largest > 512) return 1024;
-    if (2 * n_items <= 3 * (int64_t)m->n_cu && largest > 2048) return 1024;
+    if (2 * n_items <= 3 * (int64_t)m->n_cu && largest > 2048 && 3 * largest > 4 * sessions / n_items) return 1024;
     if (n_items >= 4 * (int64_t)m->n_cu && grad_lds_bytes(m) <= 20000) return 256;
     return 512;
 }
