@@ -77,9 +77,10 @@ void choose_shape(mc_model* m, int64_t n, bool uneven) {
     }
 }
 
-// Entries of the widest window: with the default item window a group of more
-// entries gets a window of its own as long as two workgroups fit a CU's LDS;
-// one 64-bit atomic to L2 per shown document otherwise bounds its items.  1M
+// Entries of the widest window: with the automatic item window a group of more
+// entries gets a window of its own, of up to 78 KB of LDS.  Two workgroups
+// then fit a CU's 160 KB (one, of the PBM's widest seventy entries, whose
+// static slots take 3 KB more); one 64-bit atomic to L2 per shown document otherwise bounds its items.  1M
 // UBM sessions on 1,500 queries of up to 1,500 documents: 432 us per
 // iteration with global atomics, 30 us with wide windows.
 int wide_window(const mc_model* m, int W) {
