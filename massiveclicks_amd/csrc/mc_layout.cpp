@@ -48,6 +48,15 @@ void choose_shape(mc_model* m, int64_t n, bool uneven) {
     // sessions 58 (1953: 27).
     const bool small_window = m->type == MC_PBM || m->type == MC_CCM;
     if (!m->block_set) m->block = small_window && n >= 1000000 ? 256 : 512;
+    // Where the caller's window cuts the set into thousands of items of a few
+    // sessions, most of 512 lanes have none: 900,000 sessions, us per iteration
+    // with 64 / 128 / 256 / 512 lanes: windows of 16 entries CCM 309 / 465 / 824
+    // / 1703, of 64 196 / 191 / 261 / 522, of 256 66 / 58 / 67 / 116, of 512 51 /
+    // 37 / 40 / 59; DBN the same within a tenth; the UBM, whose items each clear
+    // and add up their slots, of 64 422 / 385 / 346 / 519.
+    if (!m->block_set && m->item_window_set && m->item_window > 0 && m->item_window <= 512 &&
+        m->n_qd / m->item_window >= 1024)
+        m->block = m->item_window <= 32 ? 64 : m->item_window <= 128 && m->type != MC_UBM ? 128 : 256;
     if (!m->item_sessions_set) {
         const int64_t per = m->block >= 512 ? (uneven ? 384 : n < 1000000 ? 256 : 512) : (uneven ? 512 : 1024);
         // Small uneven DBN sets: with 256 sessions an item, a wavefront holds
