@@ -113,7 +113,7 @@ struct mc_model {
     // items at win_off[b] (win_cnt[b] of them) and global items at
     // glob_off[b]; split entries of batch b at shared_off[b] in d_shared_idx.
     int32_t* d_lists = nullptr;
-    std::vector<int64_t> largest_item;         // ... of the largest item per batch, and of every batch last
+    std::vector<int64_t> largest_item;         // sessions of the largest item: per batch, then of all
     std::vector<int64_t> win_off, win_cnt, glob_off, glob_cnt, shared_off, shared_cnt;
     bool grad_ready = false;
     bool grad_cleared = false;                 // d_grad is 0 wherever no session writes it
